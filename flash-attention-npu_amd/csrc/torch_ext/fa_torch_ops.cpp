@@ -573,9 +573,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor& dout, const Tensor&
     TORCH_CHECK(softmax_lse.sizes() == at::IntArrayRef({B, H, Sq}) && softmax_lse.is_contiguous(),
                 "softmax_lse must be a contiguous (batch, nheads, seqlen_q) tensor");
     Tensor lse = softmax_lse;
-    Tensor dq = at::empty(q.sizes(), q.options());
-    Tensor dk = at::empty(k.sizes(), k.options());
-    Tensor dv = at::empty(v.sizes(), v.options());
+    // in the layout of the inputs (checked stride by stride like them), as autograd hands them on
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     Tensor sd = at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
     p.batch = (int32_t)B;
     p.seqlen_q = (int32_t)Sq;
@@ -645,9 +644,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> varlen_bwd(const Tensor& dout, const 
     const int64_t T = q.size(0), H = q.size(1);
     TORCH_CHECK(softmax_lse.sizes() == at::IntArrayRef({H, T}) && softmax_lse.is_contiguous(),
                 "mha_varlen_bwd: softmax_lse must be a contiguous (nheads, total_q) tensor");
-    Tensor dq = at::empty(q.sizes(), q.options());
-    Tensor dk = at::empty(k.sizes(), k.options());
-    Tensor dv = at::empty(v.sizes(), v.options());
+    // in the layout of the inputs (checked stride by stride like them), as autograd hands them on
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     Tensor sd = at::empty({H, T}, q.options().dtype(at::kFloat));
     p.batch = (int32_t)(cu_seqlens_q.numel() - 1);
     p.seqlen_q = (int32_t)max_seqlen_q;

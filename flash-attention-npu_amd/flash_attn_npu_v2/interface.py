@@ -28,12 +28,30 @@ def _pad8(x, head_size_og):
 def _flash_attn_forward(q, k, v, dropout_p, softmax_scale, causal, window_size_left=-1, window_size_right=-1,
                         softcap=0.0, alibi_slopes=None, return_softmax=False):
     """Reference interface_arch22.py:47-77: returns (out, softmax_lse, S_dmask, rng_state)."""
+    out, lse = _dense_fwd(q, k, v, dropout_p, softmax_scale, causal, window_size_left, window_size_right, softcap,
+                          alibi_slopes)
+    return out, lse, _no_dmask(q), torch.zeros((2,), dtype=torch.int64, device=q.device)
+
+
+# The autograd Functions call the operators through these two, without the
+# dropout state of the functions above: there is no dropout, and filling
+# rng_state is a launch of its own on every forward.
+def _no_dmask(q):
+    return torch.empty((0,), dtype=q.dtype, device=q.device)
+
+
+def _dense_fwd(q, k, v, dropout_p, softmax_scale, causal, window_size_left, window_size_right, softcap, alibi_slopes):
     q, k, v = [maybe_contiguous(x) for x in (q, k, v)]
-    out, lse = ops.fwd(q, k, v, alibi_slopes, float(dropout_p), float(softmax_scale), bool(causal),
-                       int(window_size_left), int(window_size_right), float(softcap))
-    s_dmask = torch.empty((0,), dtype=q.dtype, device=q.device)
-    rng_state = torch.zeros((2,), dtype=torch.int64, device=q.device)
-    return out, lse, s_dmask, rng_state
+    return ops.fwd(q, k, v, alibi_slopes, float(dropout_p), float(softmax_scale), bool(causal), int(window_size_left),
+                   int(window_size_right), float(softcap))
+
+
+def _varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, causal,
+                window_size_left, window_size_right, softcap, alibi_slopes, block_table=None, seqused_k=None):
+    q, k, v = [maybe_contiguous(x) for x in (q, k, v)]
+    return ops.varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, seqused_k, block_table, alibi_slopes,
+                          int(max_seqlen_q), int(max_seqlen_k), float(dropout_p), float(softmax_scale), bool(causal),
+                          int(window_size_left), int(window_size_right), float(softcap))
 
 
 def _flash_attn_varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
@@ -43,14 +61,9 @@ def _flash_attn_varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q
     """Reference interface_arch22.py:113-161."""
     if leftpad_k is not None:
         raise RuntimeError("leftpad_k is not supported")
-    q, k, v = [maybe_contiguous(x) for x in (q, k, v)]
-    out, lse = ops.varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, seqused_k, block_table, alibi_slopes,
-                              int(max_seqlen_q),
-                              int(max_seqlen_k), float(dropout_p), float(softmax_scale), bool(causal),
-                              int(window_size_left), int(window_size_right), float(softcap))
-    s_dmask = torch.empty((0,), dtype=q.dtype, device=q.device)
-    rng_state = torch.zeros((2,), dtype=torch.int64, device=q.device)
-    return out, lse, s_dmask, rng_state
+    out, lse = _varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale,
+                           causal, window_size_left, window_size_right, softcap, alibi_slopes, block_table, seqused_k)
+    return out, lse, _no_dmask(q), torch.zeros((2,), dtype=torch.int64, device=q.device)
 
 
 def _flash_attn_backward(dout, q, k, v, out, softmax_lse, dq, dk, dv, dropout_p, softmax_scale, causal,
@@ -93,12 +106,10 @@ class FlashAttnFunc(torch.autograd.Function):
             softmax_scale = q.shape[-1] ** (-0.5)
         head_size_og = q.size(3)
         q, k, v = (_pad8(x, head_size_og) for x in (q, k, v))
-        out_padded, softmax_lse, s_dmask, rng_state = _flash_attn_forward(
-            q, k, v, dropout_p, softmax_scale, causal=causal, window_size_left=window_size[0],
-            window_size_right=window_size[1], softcap=softcap, alibi_slopes=alibi_slopes,
-            return_softmax=return_softmax and dropout_p > 0)
+        out_padded, softmax_lse = _dense_fwd(q, k, v, dropout_p, softmax_scale, causal, window_size[0],
+                                             window_size[1], softcap, alibi_slopes)
         if is_grad:
-            ctx.save_for_backward(q, k, v, out_padded, softmax_lse, rng_state)
+            ctx.save_for_backward(q, k, v, out_padded, softmax_lse)
             ctx.dropout_p = dropout_p
             ctx.softmax_scale = softmax_scale
             ctx.causal = causal
@@ -107,17 +118,17 @@ class FlashAttnFunc(torch.autograd.Function):
             ctx.alibi_slopes = alibi_slopes
             ctx.deterministic = deterministic
         out = out_padded[..., :head_size_og]
-        return out if not return_softmax else (out, softmax_lse, s_dmask)
+        return out if not return_softmax else (out, softmax_lse, _no_dmask(q))
 
     @staticmethod
     def backward(ctx, dout, *args):
-        q, k, v, out, softmax_lse, rng_state = ctx.saved_tensors
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        q, k, v, out, softmax_lse = ctx.saved_tensors
         head_size_og = dout.size(3)
         dout_padded = _pad8(dout, head_size_og)
-        _flash_attn_backward(dout_padded, q, k, v, out, softmax_lse, dq, dk, dv, ctx.dropout_p, ctx.softmax_scale,
-                             ctx.causal, ctx.window_size[0], ctx.window_size[1], ctx.softcap, ctx.alibi_slopes,
-                             ctx.deterministic, rng_state=rng_state)
+        # the operator's own gradients: filling tensors of ours would copy all three
+        dq, dk, dv, _ = _flash_attn_backward(
+            dout_padded, q, k, v, out, softmax_lse, None, None, None, ctx.dropout_p, ctx.softmax_scale, ctx.causal,
+            ctx.window_size[0], ctx.window_size[1], ctx.softcap, ctx.alibi_slopes, ctx.deterministic)
         dq, dk, dv = dq[..., :head_size_og], dk[..., :head_size_og], dv[..., :head_size_og]
         return dq, dk, dv, None, None, None, None, None, None, None, None, None
 
@@ -132,14 +143,13 @@ class FlashAttnVarlenFunc(torch.autograd.Function):
             softmax_scale = q.shape[-1] ** (-0.5)
         head_size_og = q.size(-1)
         q, k, v = (_pad8(x, head_size_og) for x in (q, k, v))
-        out_padded, softmax_lse, s_dmask, rng_state = _flash_attn_varlen_forward(
-            q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale,
-            causal=causal, window_size_left=window_size[0], window_size_right=window_size[1], softcap=softcap,
-            alibi_slopes=alibi_slopes, return_softmax=return_softmax and dropout_p > 0, block_table=block_table)
+        out_padded, softmax_lse = _varlen_fwd(
+            q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, causal,
+            window_size[0], window_size[1], softcap, alibi_slopes, block_table=block_table)
         if is_grad:
             if block_table is not None:
                 raise RuntimeError("flash_attn_varlen_func has no backward with a paged k/v (block_table)")
-            ctx.save_for_backward(q, k, v, out_padded, softmax_lse, cu_seqlens_q, cu_seqlens_k, rng_state)
+            ctx.save_for_backward(q, k, v, out_padded, softmax_lse, cu_seqlens_q, cu_seqlens_k)
             ctx.dropout_p = dropout_p
             ctx.max_seqlen_q = max_seqlen_q
             ctx.max_seqlen_k = max_seqlen_k
@@ -150,18 +160,17 @@ class FlashAttnVarlenFunc(torch.autograd.Function):
             ctx.alibi_slopes = alibi_slopes
             ctx.deterministic = deterministic
         out = out_padded[..., :head_size_og]
-        return out if not return_softmax else (out, softmax_lse, s_dmask)
+        return out if not return_softmax else (out, softmax_lse, _no_dmask(q))
 
     @staticmethod
     def backward(ctx, dout, *args):
-        q, k, v, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, rng_state = ctx.saved_tensors
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        q, k, v, out, softmax_lse, cu_seqlens_q, cu_seqlens_k = ctx.saved_tensors
         head_size_og = dout.size(2)
         dout_padded = _pad8(dout, head_size_og)
-        _flash_attn_varlen_backward(dout_padded, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k,
-                                    ctx.max_seqlen_q, ctx.max_seqlen_k, ctx.dropout_p, ctx.softmax_scale, ctx.causal,
-                                    ctx.window_size[0], ctx.window_size[1], ctx.softcap, ctx.alibi_slopes,
-                                    ctx.deterministic, rng_state=rng_state)
+        dq, dk, dv, _ = _flash_attn_varlen_backward(
+            dout_padded, q, k, v, out, softmax_lse, None, None, None, cu_seqlens_q, cu_seqlens_k, ctx.max_seqlen_q,
+            ctx.max_seqlen_k, ctx.dropout_p, ctx.softmax_scale, ctx.causal, ctx.window_size[0], ctx.window_size[1],
+            ctx.softcap, ctx.alibi_slopes, ctx.deterministic)
         dq, dk, dv = dq[..., :head_size_og], dk[..., :head_size_og], dv[..., :head_size_og]
         return dq, dk, dv, None, None, None, None, None, None, None, None, None, None, None, None, None, None
 
