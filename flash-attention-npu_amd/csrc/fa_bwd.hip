@@ -27,17 +27,10 @@
 //     LDS tiles): S^T = K.Q^T and dP^T = V.dO^T with q and dout in registers,
 //     then dQ^T += K^T.dS^T with K^T by transpose reads.
 // dS and P are rounded to the input type before their MFMAs.
-#include "fa_common.h"
-#include "fa_kernel_args.h"
+#include "fa_bwd.h"
 #include "fa_udiv.h"
 
-#include <type_traits>
-
 namespace fa {
-
-namespace bw {
-constexpr int kMaxBatch = 2048;
-}  // namespace bw
 
 // Tile shapes per kernel head dim (128 or 256).
 template <int HD>
@@ -69,60 +62,6 @@ struct BwCfg {
     static constexpr int BN = HD > 128 ? 32 : 64;
     static constexpr int CPK = BN * DCH / QNT;
 };
-
-struct BwBatch {
-    int sq, sk, rows;  // query positions, keys, packed rows (sq * g)
-};
-
-__device__ __forceinline__ BwBatch bw_batch(const BwdArgs& a, int b) {
-    BwBatch r;
-    int sq = a.cu_seqlens_q ? a.cu_seqlens_q[b + 1] - a.cu_seqlens_q[b] : a.Sq;
-    int sk = a.cu_seqlens_k ? a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b] : a.Sk;
-    r.sq = min(max(sq, 0), a.Sq);
-    r.sk = min(max(sk, 0), a.Sk);
-    r.rows = r.sq * a.g;
-    return r;
-}
-
-// Per-batch item prefix in LDS (s_pref[0..B]); items(b) is the work item
-// count of batch b. Every workgroup computes the same table.
-template <int NT, class F>
-__device__ __forceinline__ int bw_prefix(const BwdArgs& a, int* s_pref, F items) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int b = tid; b < a.B; b += NT) s_pref[b + 1] = items(b);
-    __syncthreads();
-    if (wave == 0) {
-        const int seg = (a.B + 63) / 64, b0 = lane * seg;
-        int local = 0;
-        for (int k = 0; k < seg; ++k)
-            if (b0 + k < a.B) local += s_pref[b0 + k + 1];
-        int incl = local;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            int v = __shfl_up(incl, o);
-            if (lane >= o) incl += v;
-        }
-        int run = incl - local;
-        for (int k = 0; k < seg; ++k)
-            if (b0 + k < a.B) {
-                run += s_pref[b0 + k + 1];
-                s_pref[b0 + k + 1] = run;
-            }
-        if (lane == 0) s_pref[0] = 0;
-    }
-    __syncthreads();
-    return s_pref[a.B];
-}
-
-__device__ __forceinline__ int bw_find_batch(const int* s_pref, int B, int w) {
-    int bl = 0, bh = B;
-    while (bh - bl > 1) {
-        const int mid = (bl + bh) >> 1;
-        if (s_pref[mid] <= w) bl = mid;
-        else bh = mid;
-    }
-    return bl;
-}
 
 // Score in log2 units from the raw dot product x: scale, optional soft cap
 // (t returned for its derivative), optional ALiBi bias.
@@ -906,7 +845,9 @@ __global__ void __launch_bounds__(BwCfg<HD>::QNT, 1) fa_bwd_dq_kernel(BwdArgs a)
 template <int DT, int HD, bool BIAS>
 static void launch_bwd_t(const BwdArgs& a, int grid_kv, int grid_q, hipStream_t stream) {
     hipLaunchKernelGGL((fa_bwd_dq_kernel<DT, HD, BIAS>), dim3(grid_q), dim3(BwCfg<HD>::QNT), 0, stream, a);
-    if (a.chunk > 0)
+    if (HD == 128 && !BIAS && bwd_kv_takes(a))
+        launch_bwd_kv(a, DT, grid_kv, stream);
+    else if (a.chunk > 0)
         hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DT, HD, true, true>), dim3(grid_kv), dim3(BwCfg<HD>::KNT), 0, stream, a);
     else
         hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DT, HD, BIAS, false>), dim3(grid_kv), dim3(BwCfg<HD>::KNT), 0, stream, a);

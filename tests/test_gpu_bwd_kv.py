@@ -1,0 +1,62 @@
+"""GPU parity of the dK/dV kernel of the plain backward at head dims 65..128
+(64-row tiles in four LDS buffers, 128-key blocks) where its tiling can go
+wrong: fewer rows than a tile, one row more or less than whole tiles and
+blocks, few and many tiles, every group size it takes and one it does not,
+windows that hide rows at either end, head dims below 128, rows with no
+visible key, ragged batches and transposed layouts. Reference and bar are
+those of test_gpu_bwd.py."""
+import numpy as np
+import pytest
+import torch
+
+from tests.test_gpu_bwd import check, rand_inputs, run_dense, run_varlen
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sq,sk", [(1, 1), (3, 130), (16, 127), (17, 128), (63, 129), (64, 64), (65, 257), (129, 31),
+                                   (256, 256), (333, 300)])
+@pytest.mark.parametrize("h,hk", [(4, 4), (8, 2)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tile_edges(sq, sk, h, hk, causal):
+    run_dense(torch.bfloat16, 2, h, hk, sq, sk, 128, causal, seed=sq * 1000 + sk)
+
+
+@pytest.mark.parametrize("g", [1, 2, 3, 8, 16, 64])
+def test_group_sizes(g):
+    run_dense(torch.bfloat16, 1, 2 * g, 2, 45, 70, 128, True, seed=g)
+
+
+@pytest.mark.parametrize("window", [(5, 0), (40, 9), (-1, 20), (70, -1), (0, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_windows(window, dtype):
+    run_dense(dtype, 1, 4, 1, 200, 210, 128, False, window=window, seed=7)
+
+
+@pytest.mark.parametrize("d", [72, 96, 120])
+def test_head_dims(d):
+    run_dense(torch.float16, 2, 4, 2, 150, 140, d, True, seed=d, api="v3")
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_ragged(causal):
+    run_varlen(torch.bfloat16, 8, 2, [1, 200, 64, 0, 129, 17], [130, 200, 1, 40, 128, 5], 128, causal, seed=3)
+
+
+def test_layouts():
+    """Heads outside positions and a packed qkv: the same gradients, bit for bit, as contiguous copies."""
+    import flash_attn_npu_v2
+    g = torch.Generator().manual_seed(5)
+    qkv = rand_inputs((2, 100, 3, 4, 128), torch.bfloat16, g).cuda()
+    do = rand_inputs((2, 100, 4, 128), torch.bfloat16, g).cuda()
+    outer = [x.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for x in qkv.unbind(2)]
+
+    def grads(parts, dout):
+        parts = [x.detach().requires_grad_(True) for x in parts]
+        return torch.autograd.grad(flash_attn_npu_v2.flash_attn_func(*parts, causal=True), parts, dout)
+
+    want = grads([x.contiguous() for x in qkv.unbind(2)], do)
+    for parts, dout in ((outer, do.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)), (qkv.unbind(2), do)):
+        for got, w, p in zip(grads(parts, dout), want, parts):
+            assert torch.equal(got, w)
+            assert got.stride() == torch.empty_like(p).stride()
