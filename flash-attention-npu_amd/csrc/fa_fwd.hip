@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(PfCfg<HD>::NT, 1) fa_prefill_kernel(FwdArgs a)
     // loop-invariant LDS offsets (elements)
     int offk[KSTEPS];
 #pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) offk[s] = li * D + (swzk(li, G * KSTEPS + s) << 3);
+    for (int s = 0; s < KSTEPS; ++s) offk[s] = li * D + (swzk(li, 4 * s + G) << 3);
     const int r4 = li >> 2, c4 = li & 3;
     int offv[DBLK];
 #pragma unroll
@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(PfCfg<HD>::NT, 1) fa_prefill_kernel(FwdArgs a)
                                  : qp + (int64_t)b * a.q_sb + (int64_t)i * a.q_si + (int64_t)h * a.q_sh;
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s)
-                qreg[rb][s] = ok && (G * KSTEPS + s) * 8 < a.hd ? widen(*reinterpret_cast<const RT*>(qrow + (G * KSTEPS + s) * 8))
+                qreg[rb][s] = ok && (4 * s + G) * 8 < a.hd ? widen(*reinterpret_cast<const RT*>(qrow + (4 * s + G) * 8))
                                                                 : u32x4{0u, 0u, 0u, 0u};
             qrows[rb] = qrow;
             qok[rb] = ok;
@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(PfCfg<HD>::NT, 1) fa_prefill_kernel(FwdArgs a)
                     const uint16_t* crow_s = static_cast<const uint16_t*>(rk->rot_sin) + (int64_t)pos * (rot_rd >> 1);
 #pragma unroll
                     for (int s = 0; s < KSTEPS; ++s)
-                        rop[rb][s] = rope_load(qrows[rb], min(G * KSTEPS + s, clast), rot_rd, INTER, crow_c, crow_s);
+                        rop[rb][s] = rope_load(qrows[rb], min(4 * s + G, clast), rot_rd, INTER, crow_c, crow_s);
                 }
                 // the first K/V tile's loads go out before the rotation, which
                 // then runs under their latency
@@ -440,7 +440,7 @@ __global__ void __launch_bounds__(PfCfg<HD>::NT, 1) fa_prefill_kernel(FwdArgs a)
                 for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                     for (int s = 0; s < KSTEPS; ++s) {
-                        const int c = G * KSTEPS + s;
+                        const int c = 4 * s + G;
                         const u32x4 rq = rope_apply<DT>(qreg[rb][s], rop[rb][s], c, rot_rd, INTER);
                         if (qok[rb] && c <= clast) qreg[rb][s] = rq;
                     }
