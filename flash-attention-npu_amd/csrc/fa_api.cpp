@@ -43,6 +43,8 @@ namespace {
 constexpr int kMaxBatch = 2048;   // sequences per attention launch (per-batch plans live in LDS)
 constexpr int kDecodeRows = 16;   // rows per (b, kv head) that take the decode kernel
 
+constexpr int kSplitKeys = 1024;  // longest keys that the pipelined prefill never splits
+
 thread_local std::string g_err;
 
 fa_status_t fail(fa_status_t st, const char* fmt, ...) {
@@ -94,6 +96,7 @@ struct Plan {
     bool rotary;
     int workers;        // decode: wave workers
     int kd;             // kernel head dim (64, 128 or 256)
+    bool pipe;          // prefill: the pipelined kernel
     size_t off_sched, off_plse, off_po, off_qrot, total;
 };
 
@@ -298,6 +301,31 @@ void make_plan(const fa_fwd_params* p, int kind, Plan& pl) {
     pl.off_po = off;
     // partial rows are written at the kernel's head dim
     if (pl.allow_split) off = align256(off + sizeof(float) * (size_t)pl.items_max * pl.BM * pl.kd);
+    pl.pipe = !pl.decode && fa::prefill_pipe_takes(p->dtype, pl.kd, p->softmax_scale, p->softcap, p->alibi_slopes != nullptr,
+                                              p->k_row_stride, p->v_row_stride, p->block_table != nullptr, p->page_block_size);
+    if (pl.pipe) {
+        // One workgroup per CU, whatever the call. Tiles of 128 rows instead of
+        // 256 where those leave CUs without one, and a split of the keys only
+        // where a sequence can be long: a split costs a merge launch (about 9
+        // us) and its partial rows, a tile of 64 keys about 1 us. us, with the
+        // 256-row tiles and 128-key chunks before: dense causal B2 S512 H16 D128
+        // 34.5 -> 20.4, B1 S1024 H16 49 -> 27, B1 S2048 H8 58 -> 37; 64 new rows
+        // onto 4096 keys, H32/8, 58 -> 31. The scratch above, sized for the
+        // larger tiles and the shorter chunks, covers either.
+        const int64_t full = (int64_t)pb * pl.hk_eff * pl.mt_max;
+        if (full < cus) {
+            pl.BM /= 2;
+            pl.mt_max = std::max(1, (pl.rows_max + pl.BM - 1) / pl.BM);
+        }
+        const int64_t base = (int64_t)pb * pl.hk_eff * pl.mt_max;
+        const int keys = kind == FA_KIND_VARLEN && !p->block_table ? p->seqlen_k : pl.kv_capacity;
+        if (p->num_splits == 0 && keys <= kSplitKeys) pl.allow_split = false;
+        pl.min_chunk = kSplitKeys / 2;
+        pl.target_items = cus;
+        if (pl.allow_split || !p->cu_seqlens_q) pl.grid = cus;
+        else pl.grid = (int)std::min<int64_t>(base, INT_MAX);
+        if (!pl.allow_split) pl.grid = (int)std::min<int64_t>(pl.grid, base);
+    }
     pl.off_qrot = off;
     // decode reads a rotated copy of q; prefill rotates q as it loads it
     const int64_t q_rows = (kind == FA_KIND_KVCACHE && p->cu_seqlens_q) ? p->total_q : (int64_t)p->batch * p->seqlen_q;
@@ -542,6 +570,8 @@ fa_status_t run_forward_ws(const fa_fwd_params* p, int kind, void* stream_v, voi
         a.target_items = pl.target_items;
         a.min_chunk = pl.min_chunk;
         a.mt_max = pl.mt_max;
+        a.tile_rows = pl.BM;
+        a.pipe = pl.pipe ? 1 : 0;
         a.page_shift = -1;
         if (paged && (p->page_block_size & (p->page_block_size - 1)) == 0) {
             int sh = 0;

@@ -27,11 +27,10 @@
 // backward 2165 -> 1830 us. Its MFMAs alone (no vector work, LDS reads, loads)
 // take 650 us at 1.8 GHz, the power limit; the clock is 1.9 GHz with all of it.
 #include "fa_bwd.h"
+#include "fa_pipe.h"
 
 namespace fa {
 namespace {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int D = 128, DCH = 16, NT = 256, BK = 128, BQ = 64;
 constexpr int KS = D / 16;                 // 16-dim steps of S and dP
@@ -44,29 +43,6 @@ constexpr int TILE = 2 * QT + 2 * ST + RAW;  // q, dout, -lse, -dsum, raw lse an
 constexpr int NBUF = 4;
 constexpr int DMA = 2 * CPQ + 1;           // loads of a wave per tile
 
-template <int DT>
-__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-    if constexpr (DT == DT_FP16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float x, float y) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    if constexpr (DT == DT_FP16) {
-        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), f16x2));
-    } else {
-        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), bf16x2));
-    }
-}
-
-// 16-byte chunk slot of chunk c in row r
-__device__ __forceinline__ int swz(int r, int c) { return c ^ (((r & 3) << 2) | ((r >> 2) & 3)); }
-
 // v as the sum of three bf16 values (exact), the first three slots of an operand row
 __device__ __forceinline__ u32x2 split3(float v) {
     const uint32_t h = f32_to_16<DT_BF16>(v);
@@ -76,44 +52,6 @@ __device__ __forceinline__ u32x2 split3(float v) {
     const uint32_t l = f32_to_16<DT_BF16>(r2);
     return u32x2{h | (m << 16), l};
 }
-
-__device__ __forceinline__ u32x4 tr_read(unsigned lo, unsigned hi) {
-    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(size_t)lo));
-    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(size_t)hi));
-    return u32x4{a[0], a[1], b[0], b[1]};
-}
-__device__ __forceinline__ u32x4 row_read(unsigned a) {
-    return *(const __attribute__((address_space(3))) u32x4*)(size_t)a;
-}
-__device__ __forceinline__ float float_read(unsigned a) {
-    return *(const __attribute__((address_space(3))) float*)(size_t)a;
-}
-// Loads straight into LDS: 16 bytes per lane from base + off[u] to the LDS
-// address lds + 1024 u + 16 lane (u < 4; 4 bytes to lds + 4 lane). The
-// instruction's offset moves both addresses, so off[u] holds (3 - u) KB more
-// and `base` is 3 KB less. In assembly, because the compiler would wait for
-// every such load before any LDS read; wait_loads<N> waits until all but the
-// wave's last N are there.
-__device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const unsigned (&off)[4]) {
-    asm volatile(
-        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %2, %1\n\t"
-        "global_load_lds_dwordx4 %3, %1 offset:1024\n\t"
-        "global_load_lds_dwordx4 %4, %1 offset:2048\n\t"
-        "global_load_lds_dwordx4 %5, %1 offset:3072" ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3])
-        : "memory");
-}
-__device__ __forceinline__ void dma4(unsigned lds, const char* base, unsigned off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %2, %1" ::"s"(lds), "s"(base), "v"(off) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
-}
-__device__ __forceinline__ void row_write(unsigned a, u32x4 v) {
-    *(__attribute__((address_space(3))) u32x4*)(size_t)a = v;
-}
-__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 
 template <int DT>
 __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {

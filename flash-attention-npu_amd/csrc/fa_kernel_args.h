@@ -87,7 +87,20 @@ struct FwdArgs {
     // of a kv head share its row tiles (Hk, g as given), g when each query
     // head has its own (Hk = H, g = 1)
     int kvdiv;
+    int tile_rows;      // prefill: packed rows per work tile
+    int pipe;           // prefill: runs on the pipelined kernel (prefill_pipe_takes)
 };
+
+// Which prefill calls run on the pipelined kernel (fa_fwd_pipe.hip); the others
+// keep the kernel of fa_fwd.hip. d: kernel head dim; dtype 0 / 1: fp16 / bf16.
+// The rows of a 64-key tile have 32-bit byte offsets, and a paged tile lies in
+// one page.
+inline bool prefill_pipe_takes(int dtype, int d, float scale, float softcap, bool alibi, int64_t k_si, int64_t v_si,
+                               bool paged, int page) {
+    auto fits = [](int64_t si) { return si >= 0 && si < (1 << 23); };
+    return d == 128 && (dtype == 0 || dtype == 1) && scale > 0.f && softcap == 0.f && !alibi && fits(k_si) &&
+           fits(v_si) && (!paged || page % 64 == 0);
+}
 
 // Backward (dense / varlen). Row layouts as in FwdArgs; lse and dsum share
 // one layout: (B,H,Sq): b*lse_sb + h*lse_sh + i; varlen (H,T): h*lse_sh + cu_q[b] + i.

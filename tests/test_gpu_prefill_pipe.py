@@ -1,0 +1,126 @@
+"""GPU parity of the pipelined prefill kernel where its tiling can go wrong:
+row tiles of 128 and 256 and key tiles of 64 met, missed by one and undershot,
+row blocks of the last wave empty, every window edge inside and between tiles,
+paged caches at the smallest page it takes and one it does not, splits of the
+keys (whole and forced) and none, ragged batches, head dims below 128, scores
+that move the running maximum late. Reference and bar are those of the forward
+oracle tests."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import fa_oracle as orc
+from tests._util import assert_close_lse, assert_close_out, bits, odt
+
+pytestmark = pytest.mark.gpu
+NT = 16
+
+
+def inputs(seed, dtype, *shapes, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return [(torch.randn(s, generator=g) * scale).to(dtype) for s in shapes]
+
+
+def dense(dtype, B, H, Hk, Sq, Sk, D, causal=False, window=(-1, -1), softcap=0.0, seed=0, grow=False):
+    import flash_attn_npu_v2
+    print(f"case pipe dense {dtype} B{B} H{H}/{Hk} {Sq}x{Sk} D{D} causal={causal} window={window} softcap={softcap}", flush=True)
+    q, k, v = inputs(seed, dtype, (B, Sq, H, D), (B, Sk, Hk, D), (B, Sk, Hk, D))
+    if grow:  # later keys score higher, so the running maximum moves again and again
+        k = (k.float() * torch.linspace(0.1, 6.0, Sk)[None, :, None, None]).to(dtype)
+    out, lse, _ = flash_attn_npu_v2.flash_attn_func(q.cuda(), k.cuda(), v.cuda(), causal=causal, window_size=window,
+                                                    softcap=softcap, return_attn_probs=True)
+    ro, rl = orc.attention(bits(q), bits(k), bits(v), dtype=odt(dtype), scale=D ** -0.5, softcap=softcap, causal=causal,
+                           window=window, nthreads=NT)
+    assert_close_out(out, ro, dtype)
+    assert_close_lse(lse, rl)
+
+
+@pytest.mark.parametrize("sq,sk", [(1, 1), (5, 64), (31, 65), (128, 63), (129, 129), (257, 128), (300, 1000), (64, 1025)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tile_edges(sq, sk, d, causal):
+    dense(torch.bfloat16, 2, 6, 2, sq, sk, d, causal, seed=sq + sk)
+
+
+@pytest.mark.parametrize("b,sq", [(1, 700), (24, 600)])  # row tiles of the small and of the large kind
+@pytest.mark.parametrize("d", [40, 72, 96, 160])
+def test_head_dims(b, sq, d):
+    dense(torch.float16, b, 4, 4, sq, 130, d, seed=d)
+
+
+@pytest.mark.parametrize("window", [(0, 0), (63, 0), (64, 3), (100, -1), (-1, 70)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_windows(window, d):
+    dense(torch.float16, 1, 4, 2, 260, 300, d, window=window, seed=9)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_rising_scores(d, softcap):
+    dense(torch.bfloat16, 1, 2, 2, 200, 700, d, causal=True, softcap=softcap, seed=4, grow=True)
+
+
+def kvcache(dtype, B, H, Hk, Sq, lens, D, page, num_splits=0, window=(-1, -1), rotary=False, seed=0):
+    import flash_attn_npu_v2
+    print(f"case pipe kvcache {dtype} B{B} H{H}/{Hk} Sq{Sq} lens={lens} D{D} page={page} splits={num_splits}", flush=True)
+    g = torch.Generator().manual_seed(seed)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    new = Sq if rotary else 0
+    cap = max(lens) + new
+    bt = None
+    if page:
+        nb = -(-cap // page)
+        bt = torch.randperm(B * nb + 2, generator=g)[:B * nb].view(B, nb).to(torch.int32)
+        kv = (B * nb + 2, page, Hk, D)
+    else:
+        kv = (B, cap, Hk, D)
+    q, kc, vc, kn, vn = inputs(seed, dtype, (B, Sq, H, D), kv, kv, (B, Sq, Hk, D), (B, Sq, Hk, D))
+    more, ref = {}, {}
+    if rotary:
+        ang = torch.arange(cap)[:, None] * 10000.0 ** (-torch.arange(0, D, 2) / D)
+        cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+        more = dict(k=kn.cuda(), v=vn.cuda(), rotary_cos=cos.cuda(), rotary_sin=sin.cuda(), rotary_interleaved=False)
+        ref = dict(k=bits(kn), v=bits(vn), rotary_cos=bits(cos), rotary_sin=bits(sin), rotary_interleaved=False)
+    kd, vd = kc.cuda(), vc.cuda()
+    out, lse = flash_attn_npu_v2.flash_attn_with_kvcache(
+        q.cuda(), kd, vd, cache_seqlens=sl.cuda(), block_table=None if bt is None else bt.cuda(), causal=True,
+        window_size=window, num_splits=num_splits, return_softmax_lse=True, **more)
+    ro, rl, rk, _ = orc.kvcache_forward(bits(q), bits(kc), bits(vc), dtype=odt(dtype), cache_seqlens=sl.numpy(),
+                                        block_table=None if bt is None else bt.numpy(), causal=True, window=window, **ref)
+    assert_close_out(out, ro, dtype)
+    assert_close_lse(lse, rl)
+    assert np.array_equal(bits(kd), rk)
+
+
+@pytest.mark.parametrize("page", [0, 16, 64, 192])
+@pytest.mark.parametrize("num_splits", [0, 1, 3])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_split_and_paged(page, num_splits, d):
+    kvcache(torch.bfloat16, 2, 8, 2, 70, [1500, 333], d, page, num_splits, seed=page + num_splits)
+
+
+@pytest.mark.parametrize("page", [0, 64])
+def test_paged_window(page):
+    kvcache(torch.bfloat16, 1, 8, 2, 90, [900], 128, page, window=(130, 0), seed=1)
+
+
+@pytest.mark.parametrize("page", [0, 128])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_rotary(page, d):
+    kvcache(torch.bfloat16, 2, 8, 2, 100, [37, 250], d, page, rotary=True, seed=2)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_ragged(causal, d):
+    import flash_attn_npu_v3
+    lens = [1, 300, 0, 64, 129, 700]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    q, k, v = inputs(3, torch.bfloat16, (cu[-1], 4, d), (cu[-1], 2, d), (cu[-1], 2, d))
+    c = torch.from_numpy(cu).cuda()
+    out, lse = flash_attn_npu_v3.flash_attn_varlen_func(q.cuda(), k.cuda(), v.cuda(), c, c, 700, 700, causal=causal,
+                                                        return_attn_probs=True)
+    ro, rl = orc.attention(bits(q), bits(k), bits(v), dtype=orc.BF16, scale=d ** -0.5, causal=causal, cu_seqlens_q=cu,
+                           cu_seqlens_k=cu, max_seqlen_q=700, nthreads=NT)
+    assert_close_out(out, ro, torch.bfloat16)
+    assert_close_lse(lse, rl)
