@@ -302,21 +302,25 @@ void make_plan(const fa_fwd_params* p, int kind, Plan& pl) {
     // partial rows are written at the kernel's head dim
     if (pl.allow_split) off = align256(off + sizeof(float) * (size_t)pl.items_max * pl.BM * pl.kd);
     pl.pipe = !pl.decode && fa::prefill_pipe_takes(p->dtype, pl.kd, p->softmax_scale, p->softcap, p->alibi_slopes != nullptr,
-                                              p->k_row_stride, p->v_row_stride, p->block_table != nullptr, p->page_block_size);
+                                              pl.rotary, p->k_row_stride, p->v_row_stride, p->block_table != nullptr, p->page_block_size);
     if (pl.pipe) {
         // One workgroup per CU, whatever the call. Tiles of 128 rows instead of
-        // 256 where those leave CUs without one, and a split of the keys only
+        // 256 where the smaller ones fill the CUs better (dense causal B3 S700
+        // H16/4 32 -> 23 us; B4 S4096 H32/8 with them 523 -> 632), and a split of the keys only
         // where a sequence can be long: a split costs a merge launch (about 9
         // us) and its partial rows, a tile of 64 keys about 1 us. us, with the
         // 256-row tiles and 128-key chunks before: dense causal B2 S512 H16 D128
         // 34.5 -> 20.4, B1 S1024 H16 49 -> 27, B1 S2048 H8 58 -> 37; 64 new rows
         // onto 4096 keys, H32/8, 58 -> 31. The scratch above, sized for the
         // larger tiles and the shorter chunks, covers either.
-        const int64_t full = (int64_t)pb * pl.hk_eff * pl.mt_max;
-        if (full < cus) {
-            pl.BM /= 2;
-            pl.mt_max = std::max(1, (pl.rows_max + pl.BM - 1) / pl.BM);
-        }
+        auto tiles = [&](int bm) -> int64_t {  // items of a call with tiles of bm rows (ragged: about)
+            if (p->cu_seqlens_q) return ((int64_t)p->total_q * pl.g / bm + pb / 2 + 1) * pl.hk_eff;
+            return (int64_t)pb * pl.hk_eff * ((pl.rows_max + bm - 1) / bm);
+        };
+        // a row of a 128-row tile costs about 9 / 8 of one of a 256-row tile
+        auto cost = [&](int bm, int rate) { return std::max<int64_t>(tiles(bm), cus) * bm * rate; };
+        pl.BM = pl.kd == 256 || cost(128, 9) < cost(256, 8) ? 128 : 256;
+        pl.mt_max = std::max(1, (pl.rows_max + pl.BM - 1) / pl.BM);
         const int64_t base = (int64_t)pb * pl.hk_eff * pl.mt_max;
         const int keys = kind == FA_KIND_VARLEN && !p->block_table ? p->seqlen_k : pl.kv_capacity;
         if (p->num_splits == 0 && keys <= kSplitKeys) pl.allow_split = false;

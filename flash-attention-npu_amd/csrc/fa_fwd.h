@@ -129,7 +129,9 @@ __device__ void build_schedule(const FwdArgs& a, int* s_pref, long long* s_red, 
     }
 }
 
-// The pipelined prefill (fa_fwd_pipe.hip)
-void launch_prefill_pipe(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
+// The pipelined prefill (fa_fwd_pipe.h) by kernel head dim
+void launch_prefill_pipe64(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
+void launch_prefill_pipe128(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
+void launch_prefill_pipe256(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
 
 }  // namespace fa

@@ -647,7 +647,9 @@ static void launch_prefill_d(const FwdArgs& a, int dtype, int grid, hipStream_t 
 
 // d: the kernel head dim, 64, 128 or 256 (a.hd <= d is the head dim in memory)
 hipError_t launch_fwd(const FwdArgs& a, int dtype, int d, int grid, hipStream_t stream) {
-    if (a.pipe) launch_prefill_pipe(a, dtype, grid, stream);
+    if (a.pipe && d == 64) launch_prefill_pipe64(a, dtype, grid, stream);
+    else if (a.pipe && d == 128) launch_prefill_pipe128(a, dtype, grid, stream);
+    else if (a.pipe) launch_prefill_pipe256(a, dtype, grid, stream);
     else if (d == 64) launch_prefill_d<64>(a, dtype, grid, stream);
     else if (d == 128) launch_prefill_d<128>(a, dtype, grid, stream);
     else if (d == 256) launch_prefill_d<256>(a, dtype, grid, stream);
@@ -665,7 +667,9 @@ static void launch_merge_d(const FwdArgs& a, int dtype, hipStream_t stream) {
 }
 
 hipError_t launch_merge(const FwdArgs& a, int dtype, int d, hipStream_t stream) {
-    if (d == 64) launch_merge_d<64>(a, dtype, stream);
+    if (d == 64 && a.tile_rows == 128) launch_merge_d<64, 128>(a, dtype, stream);
+    else if (d == 64 && a.tile_rows == 256) launch_merge_d<64, 256>(a, dtype, stream);
+    else if (d == 64) launch_merge_d<64>(a, dtype, stream);
     else if (d == 128 && a.tile_rows == 128) launch_merge_d<128, 128>(a, dtype, stream);
     else if (d == 128) launch_merge_d<128>(a, dtype, stream);
     else if (d == 256) launch_merge_d<256>(a, dtype, stream);

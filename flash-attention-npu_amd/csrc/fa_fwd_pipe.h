@@ -1,4 +1,5 @@
-// fa_fwd_pipe.hip -- the prefill forward with one wave per SIMD.
+// fa_fwd_pipe.h -- the prefill forward with one wave per SIMD (compiled per head
+// dim by fa_fwd_pipe64 / 128 / 256.hip).
 //
 // The work items, masks and split of fa_fwd.hip; another inner loop. Four waves
 // of RB x 32 packed rows; K and V tiles go straight from memory into four LDS
@@ -18,15 +19,26 @@
 // 8192^3 matrix product reaches 1.24 on this card), causal 593 -> 540; chunked
 // prefill B4 2048 onto 6144 895 -> 813, with rotary and append 953 -> 860.
 // Without the softmax 785 us, with products alone 730 (of 920, another box).
+// Head dim 256 (32 rows per wave, 32-key tiles), window 1024 and soft cap, B2 S4096
+// H16/8: 281 -> 190 us; head dim 64 (bound by the softmax, whose share of the
+// products is twice as large), B8 S1025 H16 fp16: 102 -> 97.
+#pragma once
 #include "fa_fwd.h"
 #include "fa_pipe.h"
 #include "fa_rope.h"
 
 namespace fa {
-namespace {
+namespace pipe {
 
 constexpr int NT = 256, NBUF = 4;
 constexpr float kLazy = 8.f;  // log2 headroom before the running maximum moves
+
+// Slot of chunk c in row r: fa_pipe.h's; 128-byte rows (two to a line of LDS
+// banks) take theirs from the row pair, conflict free for the same reads.
+template <int HD>
+__device__ __forceinline__ int slot_of(int r, int c) {
+    return HD == 64 ? c ^ ((((r >> 1) & 1) << 2) | ((r >> 2) & 3)) : swz(r, c);
+}
 
 template <int HD, int RBLK>
 struct PipeCfg {
@@ -43,7 +55,8 @@ struct PipeCfg {
     static constexpr int TILE = 2 * KT;
 };
 
-template <int DT, int HD, int RBLK, bool PAGED, bool ROT>
+// CAP: soft cap (scores are capped and in log2 units once their maximum is taken)
+template <int DT, int HD, int RBLK, bool PAGED, bool ROT, bool CAP>
 __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
     using C = PipeCfg<HD, RBLK>;
     constexpr int RB = C::RB, BM = C::BM, BN = C::BN, NH = C::NH, KS = C::KS, DB = C::DB, CH = C::CH, ROW = C::ROW,
@@ -60,13 +73,15 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
     build_schedule<BM, C::BN, NT, 4>(a, s_pref, s_red, total, chunk_auto);
 
     const unsigned lds0 = lds_addr(s_t);
-    const unsigned rowa = lds0 + col * ROW + (swz(col, hi) << 4);  // chunk 2s + hi: ^ (s << 5)
+    const unsigned rowa = lds0 + col * ROW + (slot_of<HD>(col, hi) << 4);  // chunk 2s + hi: ^ (s << 5)
     const int tr_r = 4 * hi + ((lane & 15) >> 2), tr_c = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-    const unsigned tra = lds0 + KT + tr_r * ROW + (swz(tr_r, tr_c) << 4) + (lane & 1) * 8;  // dim block db: ^ (db << 6)
+    const unsigned tra = lds0 + KT + tr_r * ROW + (slot_of<HD>(tr_r, tr_c) << 4) + (lane & 1) * 8;  // dim block db: ^ (db << 6)
 
     const uint16_t* qp = static_cast<const uint16_t*>(a.q);
     uint16_t* op = static_cast<uint16_t*>(a.out);
-    const float cs = a.scale_log2;
+    const float cs = CAP ? 1.f : a.scale_log2;
+    // cap * tanh(scale s / cap) in log2 units = c1 - 2 c1 / (2^(c0 s) + 1)
+    [[maybe_unused]] const float c0 = CAP ? 2.f * a.scale_log2 / a.softcap : 0.f, c1 = a.softcap * kLog2e;
 
     for (int k = 0; k * (int)gridDim.x < total; ++k) {
         const int w = k * (int)gridDim.x + ((k & 1) ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x);
@@ -128,7 +143,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int r = C::RPL * (4 * wave + u) + lane / CH;
-            const int c = min(swz(r, lane % CH), (a.hd >> 3) - 1);  // chunks past the head dim: q is 0 there
+            const int c = min(slot_of<HD>(r, lane % CH), (a.hd >> 3) - 1);  // chunks past the head dim: q is 0 there
             const int rl = min(r, k_hi - 1 - base - (ntiles - 1) * BN);
             ko[0][u] = 2u * (unsigned)(r * (int)a.k_si + c * 8) + (3 - u) * 1024;
             vo[0][u] = 2u * (unsigned)(r * (int)a.v_si + c * 8) + (3 - u) * 1024;
@@ -280,6 +295,9 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
         };
 
         float peak[RB];
+        [[maybe_unused]] auto cap = [&](float x) {
+            return __builtin_fmaf(-2.f * c1, __builtin_amdgcn_rcpf(fast_exp2(x * c0) + 1.f), c1);
+        };
         auto visible = [&](f32x16 (&ns_)[RB], int e, int s0) {  // s0: key offset of the half
             const int rb = e / 16, i = e % 16, j = s0 + 8 * (i / 4) + i % 4;
             ns_[rb][i] = j >= rlo[rb] && j <= rhi[rb] ? ns_[rb][i] : -INFINITY;
@@ -331,6 +349,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
                 for (int e = 0; e < NE; ++e) {
                     if (slot != SS + 2 + e * (2 * SP - 4) / NE) continue;
+                    if constexpr (CAP) n_[e / 16][e % 16] = cap(n_[e / 16][e % 16]);
                     if constexpr (decltype(mask)::value) visible(n_, e, s0n);
                     if (e % 16 == 0) peak[e / 16] = n_[e / 16][0];
                     else peak[e / 16] = fmaxf(peak[e / 16], n_[e / 16][e % 16]);
@@ -372,7 +391,6 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 
         if (ntiles > 0) {
             using H0 = std::integral_constant<int, 0>;
-            using H1 = std::integral_constant<int, 1>;
             wait_loads<0>();  // (with the q rows, which the compiler waits for)
             __syncthreads();
             f32x16 s0[RB], s1[RB];
@@ -386,6 +404,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             }
 #pragma unroll
             for (int e = 0; e < NE; ++e) {
+                if constexpr (CAP) s0[e / 16][e % 16] = cap(s0[e / 16][e % 16]);
                 visible(s0, e, 0);
                 if (e % 16 == 0) peak[e / 16] = s0[e / 16][0];
                 else peak[e / 16] = fmaxf(peak[e / 16], s0[e / 16][e % 16]);
@@ -395,7 +414,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
                 for (int s = 0; s < KS; ++s) move_on(ra[s], TILE);
             }
-            read_rows(NH - 1, 0);
+            read_rows(NH > 1 ? 1 : 0, 0);
             int t = 0, nb = 1, fb = 3;  // buffers of tiles t + 1 and t + 3
             auto next_buf = [](int x) { return x == NBUF - 1 ? 0 : x + 1; };
             auto step_to = [](int x) { return x == 0 ? 0u - (NBUF - 1) * (unsigned)TILE : (unsigned)TILE; };
@@ -404,32 +423,38 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             auto tile = [&](auto mask) {
                 const unsigned by = step_to(nb);  // from tile t's buffer to the next
                 const int s0k = t * BN;
-                if constexpr (NH == 2) {
-                    unit(s0, s1, H1{}, H0{}, s0k + 32, mask,
-                         [&](int x) {
-                             if (x == SP / 2) {
+                if constexpr (NH > 1) {
+                    auto half = [&](auto hh) {  // the next unit's scores: half (h + 1) % NH, the one's after it (h + 2) % NH
+                        constexpr int H = decltype(hh)::value;
+                        unit(H % 2 ? s1 : s0, H % 2 ? s0 : s1, std::integral_constant<int, (H + 1) % NH>{}, hh,
+                             s0k + 32 * (H + 1), mask,
+                             [&](int x) {
+                                 if (H == NH - 2 && x == SP / 2) {
 #pragma unroll
-                                 for (int s = 0; s < KS; ++s) move_on(ra[s], by);
-                             }
-                             if (x == LAST - 1) {
-                                 wait_loads<8>();
-                                 __syncthreads();
-                             }
-                         },
-                         [&]() { read_rows(0, 0); });
-                    raise(true);
-                    unit(s1, s0, H0{}, H1{}, s0k + 64, mask,
-                         [&](int x) {
-                             if (x == 0) ask();
-                             if (x == LAST) {
-#pragma unroll
-                                 for (int db = 0; db < DB; ++db) {
-                                     move_on(ta[db], by);
-                                     move_on(tb[db], by);
+                                     for (int s = 0; s < KS; ++s) move_on(ra[s], by);
                                  }
-                             }
-                         },
-                         [&]() { read_rows(1, 0); });
+                                 if (H == NH - 2 && x == LAST - 1) {
+                                     wait_loads<8>();
+                                     __syncthreads();
+                                 }
+                                 if (H == NH - 1 && x == 0) ask();
+                                 if (H == NH - 1 && x == LAST) {
+#pragma unroll
+                                     for (int db = 0; db < DB; ++db) {
+                                         move_on(ta[db], by);
+                                         move_on(tb[db], by);
+                                     }
+                                 }
+                             },
+                             [&]() { read_rows((H + 2) % NH, 0); });
+                        if constexpr (H < NH - 1) raise(true);
+                    };
+                    half(std::integral_constant<int, 0>{});
+                    half(std::integral_constant<int, 1>{});
+                    if constexpr (NH == 4) {
+                        half(std::integral_constant<int, 2>{});
+                        half(std::integral_constant<int, 3>{});
+                    }
                 } else {
                     const unsigned by2 = step_to(next_buf(nb));  // from tile t + 1's buffer to the next
                     unit(s0, s1, H0{}, H0{}, s0k + 32, mask,
@@ -516,25 +541,24 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 
 template <int DT, int HD, int RB>
 void launch_t(const FwdArgs& a, int grid, hipStream_t stream) {
-    if (a.block_table) {
-        if (a.rot_cos) hipLaunchKernelGGL((fa_prefill_pipe_kernel<DT, HD, RB, true, true>), dim3(grid), dim3(NT), 0, stream, a);
-        else hipLaunchKernelGGL((fa_prefill_pipe_kernel<DT, HD, RB, true, false>), dim3(grid), dim3(NT), 0, stream, a);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, a); };
+    if (a.softcap > 0.f) {
+        if (a.block_table) go(fa_prefill_pipe_kernel<DT, HD, RB, true, false, true>);
+        else go(fa_prefill_pipe_kernel<DT, HD, RB, false, false, true>);
+    } else if (a.block_table) {
+        if (a.rot_cos) go(fa_prefill_pipe_kernel<DT, HD, RB, true, true, false>);
+        else go(fa_prefill_pipe_kernel<DT, HD, RB, true, false, false>);
     } else {
-        if (a.rot_cos) hipLaunchKernelGGL((fa_prefill_pipe_kernel<DT, HD, RB, false, true>), dim3(grid), dim3(NT), 0, stream, a);
-        else hipLaunchKernelGGL((fa_prefill_pipe_kernel<DT, HD, RB, false, false>), dim3(grid), dim3(NT), 0, stream, a);
+        if (a.rot_cos) go(fa_prefill_pipe_kernel<DT, HD, RB, false, true, false>);
+        else go(fa_prefill_pipe_kernel<DT, HD, RB, false, false, false>);
     }
 }
 
-}  // namespace
-
-void launch_prefill_pipe(const FwdArgs& a, int dtype, int grid, hipStream_t stream) {
-    if (dtype == DT_BF16) {
-        if (a.tile_rows == 128) launch_t<DT_BF16, 128, 1>(a, grid, stream);
-        else launch_t<DT_BF16, 128, 2>(a, grid, stream);
-    } else {
-        if (a.tile_rows == 128) launch_t<DT_FP16, 128, 1>(a, grid, stream);
-        else launch_t<DT_FP16, 128, 2>(a, grid, stream);
-    }
+template <int HD, int RB>
+void launch_d(const FwdArgs& a, int dtype, int grid, hipStream_t stream) {
+    if (dtype == DT_BF16) launch_t<DT_BF16, HD, RB>(a, grid, stream);
+    else launch_t<DT_FP16, HD, RB>(a, grid, stream);
 }
 
+}  // namespace pipe
 }  // namespace fa

@@ -91,15 +91,15 @@ struct FwdArgs {
     int pipe;           // prefill: runs on the pipelined kernel (prefill_pipe_takes)
 };
 
-// Which prefill calls run on the pipelined kernel (fa_fwd_pipe.hip); the others
+// Which prefill calls run on the pipelined kernel (fa_fwd_pipe.h); the others
 // keep the kernel of fa_fwd.hip. d: kernel head dim; dtype 0 / 1: fp16 / bf16.
-// The rows of a 64-key tile have 32-bit byte offsets, and a paged tile lies in
+// The rows of a tile (16 KB) have 32-bit byte offsets, and a paged tile lies in
 // one page.
-inline bool prefill_pipe_takes(int dtype, int d, float scale, float softcap, bool alibi, int64_t k_si, int64_t v_si,
-                               bool paged, int page) {
-    auto fits = [](int64_t si) { return si >= 0 && si < (1 << 23); };
-    return d == 128 && (dtype == 0 || dtype == 1) && scale > 0.f && softcap == 0.f && !alibi && fits(k_si) &&
-           fits(v_si) && (!paged || page % 64 == 0);
+inline bool prefill_pipe_takes(int dtype, int d, float scale, float softcap, bool alibi, bool rotary, int64_t k_si,
+                               int64_t v_si, bool paged, int page) {
+    auto fits = [](int64_t si) { return si >= 0 && si < (1 << 22); };
+    return (dtype == 0 || dtype == 1) && scale > 0.f && !alibi && !(softcap > 0.f && rotary) && fits(k_si) &&
+           fits(v_si) && (!paged || page % (8192 / d) == 0);
 }
 
 // Backward (dense / varlen). Row layouts as in FwdArgs; lse and dsum share
