@@ -734,8 +734,8 @@ fa_status_t run_backward(const fa_bwd_params* p, int kind, void* stream_v) {
         a.wr = wr;
         a.chunk = p->attention_chunk;
         const int64_t gkv = (int64_t)nb * p->nheads_k * (((int64_t)p->seqlen_k + fa::bwd_key_block(kd) - 1) / fa::bwd_key_block(kd));
-        const int64_t gq = (int64_t)nb * p->nheads_k *
-                           (((int64_t)p->seqlen_q * a.g + fa::bwd_row_block(kd) - 1) / fa::bwd_row_block(kd));
+        const int bm = std::min(fa::bwd_row_block(kd), 128);  // the smaller of the two dQ kernels' row tiles
+        const int64_t gq = (int64_t)nb * p->nheads_k * (((int64_t)p->seqlen_q * a.g + bm - 1) / bm);
         // the kernels walk their work items in alternating passes over the
         // grid: same-length sequences run on one workgroup per CU taking
         // several items each (B4 S4096 H32/8 causal the same as with 2 x CUs

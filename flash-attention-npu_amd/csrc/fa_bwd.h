@@ -66,6 +66,10 @@ __device__ __forceinline__ int bw_find_batch(const int* s_pref, int B, int w) {
     return bl;
 }
 
+// dQ and dsum without ALiBi or chunks (fa_bwd_dq.hip); 128-row items
+bool bwd_dq_takes(const BwdArgs& a);
+void launch_bwd_dq(const BwdArgs& a, int dtype, int d, int grid, hipStream_t stream);
+
 // dK and dV at head dims 65..128 without soft cap, ALiBi or chunks (fa_bwd_kv.hip)
 bool bwd_kv_takes(const BwdArgs& a);
 void launch_bwd_kv(const BwdArgs& a, int dtype, int grid, hipStream_t stream);

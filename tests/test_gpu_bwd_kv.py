@@ -60,3 +60,18 @@ def test_layouts():
         for got, w, p in zip(grads(parts, dout), want, parts):
             assert torch.equal(got, w)
             assert got.stride() == torch.empty_like(p).stride()
+
+
+@pytest.mark.parametrize("sq,sk", [(1, 33), (127, 64), (129, 257), (300, 31)])
+@pytest.mark.parametrize("d", [40, 64, 128, 160, 256])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_dq_tiles(sq, sk, d, softcap):
+    """The dQ kernel's 128-row items and 32- to 128-key tiles at every head dim, plain and with a soft cap."""
+    run_dense(torch.bfloat16, 1, 6, 2, sq, sk, d, True, softcap=softcap, seed=sq + d)
+
+
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("window", [(40, 9), (-1, 20), (70, -1)])
+def test_dq_windows(d, window):
+    run_dense(torch.float16, 1, 4, 1, 200, 210, d, False, window=window, softcap=15.0, seed=8)
+    run_varlen(torch.bfloat16, 8, 2, [1, 200, 64, 0, 129], [130, 200, 1, 40, 128], d, False, window=window, seed=4)
