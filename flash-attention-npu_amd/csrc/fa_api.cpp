@@ -327,7 +327,8 @@ void make_plan(const fa_fwd_params* p, int kind, Plan& pl) {
         pl.min_chunk = kSplitKeys / 2;
         pl.target_items = cus;
         if (pl.allow_split || !p->cu_seqlens_q) pl.grid = cus;
-        else pl.grid = (int)std::min<int64_t>(base, INT_MAX);
+        else  // ragged: one workgroup per item, at most a part tile per sequence more than the rows fill
+            pl.grid = (int)std::min<int64_t>({base, ((int64_t)p->total_q * pl.g / pl.BM + pb) * pl.hk_eff, INT_MAX});
         if (!pl.allow_split) pl.grid = (int)std::min<int64_t>(pl.grid, base);
     }
     pl.off_qrot = off;
@@ -740,10 +741,15 @@ fa_status_t run_backward(const fa_bwd_params* p, int kind, void* stream_v) {
         // grid: same-length sequences run on one workgroup per CU taking
         // several items each (B4 S4096 H32/8 causal the same as with 2 x CUs
         // workgroups, B2 3-4 % faster), ragged ones on one workgroup per item
-        // (up to 16 x CUs)
+        // (up to 16 x CUs), counted from the rows in all and a part item per
+        // sequence; the keys are taken to be as many as the rows, as in self
+        // attention (the kernels walk on where there are more)
         const int cap = (p->cu_seqlens_q ? 16 : 1) * cu_count();
-        const int grid_kv = (int)std::max<int64_t>(1, std::min<int64_t>(gkv, cap));
-        const int grid_q = (int)std::max<int64_t>(1, std::min<int64_t>(gq, cap));
+        auto packed = [&](int64_t items, int64_t rows, int block) {
+            return p->cu_seqlens_q ? std::min(items, (rows / block + nb) * p->nheads_k) : items;
+        };
+        const int grid_kv = (int)std::max<int64_t>(1, std::min<int64_t>(packed(gkv, p->total_q, fa::bwd_key_block(kd)), cap));
+        const int grid_q = (int)std::max<int64_t>(1, std::min<int64_t>(packed(gq, (int64_t)p->total_q * a.g, bm), cap));
         hipError_t e = fa::launch_bwd(a, p->dtype, kd, grid_kv, grid_q, static_cast<hipStream_t>(stream_v));
         if (e != hipSuccess) return fail(FA_EHIP, "backward launch failed: %s", hipGetErrorString(e));
     }

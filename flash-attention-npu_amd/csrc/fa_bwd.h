@@ -56,6 +56,33 @@ __device__ __forceinline__ int bw_prefix(const BwdArgs& a, int* s_pref, F items)
     return s_pref[a.B];
 }
 
+// The same with the sequences of a small ragged batch in order of falling item
+// count (s_ord[p]: sequence at place p of the list), so that the long ones do
+// not come last; others keep their order. s_pref then goes by place.
+constexpr int kOrdered = 64;
+template <int NT, class F>
+__device__ __forceinline__ int bw_ordered_prefix(const BwdArgs& a, int* s_pref, int* s_ord, F items) {
+    if (!a.cu_seqlens_q || a.B > kOrdered) return bw_prefix<NT>(a, s_pref, items);
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 64) {
+        const int n = lane < a.B ? items(lane) : -1;
+        int place = 0, before = 0;
+        for (int c = 0; c < a.B; ++c) {
+            const int m = __shfl(n, c);
+            const bool first = m > n || (m == n && c < lane);
+            place += first ? 1 : 0;
+            before += first ? m : 0;
+        }
+        if (lane < a.B) {
+            s_ord[place] = lane;
+            s_pref[place] = before;
+            if (place == a.B - 1) s_pref[a.B] = before + n;
+        }
+    }
+    __syncthreads();
+    return s_pref[a.B];
+}
+
 __device__ __forceinline__ int bw_find_batch(const int* s_pref, int B, int w) {
     int bl = 0, bh = B;
     while (bh - bl > 1) {

@@ -43,10 +43,10 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_dq_pipe_kernel(BwdArgs a) {
     constexpr int SS = 2 * KS * RB, SP = DB * RB;  // slots: S and dP products, then dQ's of the first and the last 16 keys
     static_assert(KT == 4 * 4 * 1024, "four loads of four waves bring a tile");
     __shared__ __attribute__((aligned(256))) char s_t[NBUF * TILE];
-    __shared__ int s_pref[bw::kMaxBatch + 1];
+    __shared__ int s_pref[bw::kMaxBatch + 1], s_ord[kOrdered];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hi = lane >> 5;
-    const int total = bw_prefix<NT>(a, s_pref, [&](int b) {
+    const int total = bw_ordered_prefix<NT>(a, s_pref, s_ord, [&](int b) {
         const BwBatch bb = bw_batch(a, b);
         return a.Hk * ((bb.rows + BM - 1) / BM);
     });
@@ -68,9 +68,10 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_dq_pipe_kernel(BwdArgs a) {
     for (int k = 0; k * (int)gridDim.x < total; ++k) {
         const int w = k * (int)gridDim.x + ((k & 1) ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x);
         if (w >= total) continue;
-        const int b = __builtin_amdgcn_readfirstlane(bw_find_batch(s_pref, a.B, w));
+        const int place = bw_find_batch(s_pref, a.B, w);
+        const int b = __builtin_amdgcn_readfirstlane(a.cu_seqlens_q && a.B <= kOrdered ? s_ord[place] : place);
         const BwBatch bb = bw_batch(a, b);
-        const int local = w - __builtin_amdgcn_readfirstlane(s_pref[b]);
+        const int local = w - __builtin_amdgcn_readfirstlane(s_pref[place]);
         const int hk = local % a.Hk;
         // heavy first: with a right window bound (causal) later row tiles see more keys
         const int nmt = (bb.rows + BM - 1) / BM;

@@ -56,10 +56,10 @@ __device__ __forceinline__ u32x2 split3(float v) {
 template <int DT>
 __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
     __shared__ __attribute__((aligned(256))) uint16_t s_t[NBUF * TILE];
-    __shared__ int s_pref[bw::kMaxBatch + 1];
+    __shared__ int s_pref[bw::kMaxBatch + 1], s_ord[kOrdered];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hi = lane >> 5;
-    const int total = bw_prefix<NT>(a, s_pref, [&](int b) {
+    const int total = bw_ordered_prefix<NT>(a, s_pref, s_ord, [&](int b) {
         const BwBatch bb = bw_batch(a, b);
         return a.Hk * ((bb.sk + BK - 1) / BK);
     });
@@ -84,9 +84,10 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
     for (int k = 0; k * (int)gridDim.x < total; ++k) {
         const int w = k * (int)gridDim.x + ((k & 1) ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x);
         if (w >= total) continue;
-        const int b = __builtin_amdgcn_readfirstlane(bw_find_batch(s_pref, a.B, w));
+        const int place = bw_find_batch(s_pref, a.B, w);
+        const int b = __builtin_amdgcn_readfirstlane(a.cu_seqlens_q && a.B <= kOrdered ? s_ord[place] : place);
         const BwBatch bb = bw_batch(a, b);
-        const int local = w - __builtin_amdgcn_readfirstlane(s_pref[b]);
+        const int local = w - __builtin_amdgcn_readfirstlane(s_pref[place]);
         const int hk = local % a.Hk;
         const int nkt = (bb.sk + BK - 1) / BK;
         const int kt = (a.wl >= 0 && a.wr < 0) ? nkt - 1 - local / a.Hk : local / a.Hk;

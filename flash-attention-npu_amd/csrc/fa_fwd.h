@@ -129,6 +129,38 @@ __device__ void build_schedule(const FwdArgs& a, int* s_pref, long long* s_red, 
     }
 }
 
+// Without a split: the item list of a small ragged batch with the sequences in
+// order of falling item count (s_ord[p]: sequence at place p of the list, by
+// which s_pref goes), so that the long ones do not come last.
+constexpr int kOrdered = 64;
+__device__ __forceinline__ bool ordered(const FwdArgs& a) { return a.cu_seqlens_q && a.B <= kOrdered && !a.allow_split; }
+template <int BM>
+__device__ int ordered_schedule(const FwdArgs& a, int* s_pref, int* s_ord) {
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 64) {
+        int n = -1;
+        if (lane < a.B) {
+            BatchInfo bi;
+            batch_info<BM>(a, lane, bi);
+            n = a.Hk * bi.mt;
+        }
+        int place = 0, before = 0;
+        for (int c = 0; c < a.B; ++c) {
+            const int m = __shfl(n, c);
+            const bool first = m > n || (m == n && c < lane);
+            place += first ? 1 : 0;
+            before += first ? m : 0;
+        }
+        if (lane < a.B) {
+            s_ord[place] = lane;
+            s_pref[place] = before;
+            if (place == a.B - 1) s_pref[a.B] = before + n;
+        }
+    }
+    __syncthreads();
+    return s_pref[a.B];
+}
+
 // The pipelined prefill (fa_fwd_pipe.h) by kernel head dim
 void launch_prefill_pipe64(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
 void launch_prefill_pipe128(const FwdArgs& a, int dtype, int grid, hipStream_t stream);

@@ -65,12 +65,13 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
     constexpr int SS = KS * RB, SP = DB * RB;
     static_assert(KT == 4 * 4 * 1024, "four loads of four waves bring a tile");
     __shared__ __attribute__((aligned(256))) char s_t[NBUF * TILE];
-    __shared__ int s_pref[kMaxBatchLds + 1];
+    __shared__ int s_pref[kMaxBatchLds + 1], s_ord[kOrdered];
     __shared__ long long s_red[8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hi = lane >> 5;
-    int total, chunk_auto;
-    build_schedule<BM, C::BN, NT, 4>(a, s_pref, s_red, total, chunk_auto);
+    int total, chunk_auto = 0;
+    if (ordered(a)) total = ordered_schedule<BM>(a, s_pref, s_ord);
+    else build_schedule<BM, C::BN, NT, 4>(a, s_pref, s_red, total, chunk_auto);
 
     const unsigned lds0 = lds_addr(s_t);
     const unsigned rowa = lds0 + col * ROW + (slot_of<HD>(col, hi) << 4);  // chunk 2s + hi: ^ (s << 5)
@@ -92,12 +93,12 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             if (s_pref[mid] <= w) bl = mid;
             else bh = mid;
         }
-        const int b = __builtin_amdgcn_readfirstlane(bl);
+        const int b = __builtin_amdgcn_readfirstlane(ordered(a) ? s_ord[bl] : bl);
         BatchInfo bi;
         batch_info<BM>(a, b, bi);
         int ns, chunk;
         split_of(a, bi.hi - bi.lo, chunk_auto, ns, chunk);
-        const int local = w - __builtin_amdgcn_readfirstlane(s_pref[b]);
+        const int local = w - __builtin_amdgcn_readfirstlane(s_pref[bl]);
         const int hk = local % a.Hk;
         const int split = (local / a.Hk) % ns;
         const int mt = bi.mt - 1 - local / a.Hk / ns;  // heaviest causal tiles first
