@@ -110,6 +110,9 @@ __global__ void __launch_bounds__(BwCfg<HD>::KNT, 1) fa_bwd_dkdv_kernel(BwdArgs 
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, G = lane >> 4;
+    // 16-byte chunk of lane group G in step s: the order whose row reads of the
+    // tile have no bank conflicts (head dim 256: 2 to a bank with G * KSTEPS + s)
+    auto chunk = [&](int s) { return HD == 256 ? 4 * s + G : G * KSTEPS + s; };
     const int total = bw_prefix<NT>(a, s_pref, [&](int b) {
         const BwBatch bb = bw_batch(a, b);
         return a.Hk * ((bb.sk + BK - 1) / BK);
@@ -122,7 +125,7 @@ __global__ void __launch_bounds__(BwCfg<HD>::KNT, 1) fa_bwd_dkdv_kernel(BwdArgs 
     int offr[KSTEPS];
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s)
-        offr[s] = SPLIT ? split_addr128(li, G * KSTEPS + s, 0) : li * D + (tv(li, G * KSTEPS + s) << 3);
+        offr[s] = SPLIT ? split_addr128(li, chunk(s), 0) : li * D + (tv(li, chunk(s)) << 3);
     const int r4 = li >> 2, c4 = li & 3;
     int offt[DBLK];
 #pragma unroll
@@ -166,7 +169,7 @@ __global__ void __launch_bounds__(BwCfg<HD>::KNT, 1) fa_bwd_dkdv_kernel(BwdArgs 
             const int jl = jw + 16 * rk + li;
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) {
-                const int c = G * KSTEPS + s;
+                const int c = chunk(s);
                 const bool in = jl < bb.sk && c * 8 < a.hd;
                 kreg[rk][s] = in ? *reinterpret_cast<const u32x4*>(kp + kbase + (int64_t)jl * a.k_si + (int64_t)hk * a.k_sh + c * 8)
                                  : u32x4{0u, 0u, 0u, 0u};
