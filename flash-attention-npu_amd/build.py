@@ -28,8 +28,8 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = os.environ.get("FA_MI355X_ARCH", "gfx950")
 
 HIP_SOURCES = ["fa_fwd.hip", "fa_fwd_pipe64.hip", "fa_fwd_pipe128.hip", "fa_fwd_pipe256.hip",
-               "fa_decode.hip", "fa_kv_prep.hip", "fa_bwd.hip", "fa_bwd_kv.hip", "fa_bwd_dq.hip",
-               "fa_api.cpp", "fa_noalloc.hip"]
+               "fa_fwd_pipe_fp8.hip", "fa_decode.hip", "fa_kv_prep.hip", "fa_bwd.hip", "fa_bwd_kv.hip",
+               "fa_bwd_dq.hip", "fa_api.cpp", "fa_noalloc.hip"]
 HIPFLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     # no packed fp32 ops (v_pk_*_f32) in any generated code
@@ -57,7 +57,7 @@ def _run(cmd):
 # vector registers; without the flag each score is copied out of an
 # accumulation register and the dK/dV kernel spills 204 bytes.
 SRC_FLAGS = {
-    **{f"fa_fwd_pipe{d}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] for d in (64, 128, 256)},
+    **{f"fa_fwd_pipe{d}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] for d in (64, 128, 256, "_fp8")},
     "fa_bwd_dq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "fa_bwd_kv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "fa_fwd.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],

@@ -162,6 +162,7 @@ __device__ int ordered_schedule(const FwdArgs& a, int* s_pref, int* s_ord) {
 }
 
 // The pipelined prefill (fa_fwd_pipe.h) by kernel head dim
+void launch_prefill_pipe_fp8(const FwdArgs& a, int grid, hipStream_t stream);
 void launch_prefill_pipe64(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
 void launch_prefill_pipe128(const FwdArgs& a, int dtype, int grid, hipStream_t stream);
 void launch_prefill_pipe256(const FwdArgs& a, int dtype, int grid, hipStream_t stream);

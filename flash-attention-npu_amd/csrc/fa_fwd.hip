@@ -647,7 +647,8 @@ static void launch_prefill_d(const FwdArgs& a, int dtype, int grid, hipStream_t 
 
 // d: the kernel head dim, 64, 128 or 256 (a.hd <= d is the head dim in memory)
 hipError_t launch_fwd(const FwdArgs& a, int dtype, int d, int grid, hipStream_t stream) {
-    if (a.pipe && d == 64) launch_prefill_pipe64(a, dtype, grid, stream);
+    if (a.pipe && dtype == DT_FP8) launch_prefill_pipe_fp8(a, grid, stream);
+    else if (a.pipe && d == 64) launch_prefill_pipe64(a, dtype, grid, stream);
     else if (a.pipe && d == 128) launch_prefill_pipe128(a, dtype, grid, stream);
     else if (a.pipe) launch_prefill_pipe256(a, dtype, grid, stream);
     else if (d == 64) launch_prefill_d<64>(a, dtype, grid, stream);

@@ -35,22 +35,23 @@ constexpr float kLazy = 8.f;  // log2 headroom before the running maximum moves
 
 // Slot of chunk c in row r: fa_pipe.h's; 128-byte rows (two to a line of LDS
 // banks) take theirs from the row pair, conflict free for the same reads.
-template <int HD>
+template <int ROW>
 __device__ __forceinline__ int slot_of(int r, int c) {
-    return HD == 64 ? c ^ ((((r >> 1) & 1) << 2) | ((r >> 2) & 3)) : swz(r, c);
+    return ROW == 128 ? c ^ ((((r >> 1) & 1) << 2) | ((r >> 2) & 3)) : swz(r, c);
 }
 
-template <int HD, int RBLK>
+// EB: bytes per element of q, K and V
+template <int HD, int RBLK, int EB>
 struct PipeCfg {
     static constexpr int RB = RBLK;            // 32-row blocks per wave
     static constexpr int BM = 4 * RB * 32;     // packed rows per work tile
-    static constexpr int NH = 256 / HD;        // 32-key halves per LDS tile
+    static constexpr int ROW = EB * HD;        // bytes
+    static constexpr int NH = 512 / ROW;       // 32-key halves per LDS tile
     static constexpr int BN = 32 * NH;
-    static constexpr int KS = HD / 16;         // 16-dim steps of S
+    static constexpr int KS = ROW / 32;        // K operand reads: 16 bytes of each half wave
     static constexpr int DB = HD / 32;         // 32-dim blocks of O
-    static constexpr int CH = HD / 8;          // 16-byte chunks per row
+    static constexpr int CH = ROW / 16;        // 16-byte chunks per row
     static constexpr int RPL = 64 / CH;        // rows per LDS load
-    static constexpr int ROW = 2 * HD;         // bytes
     static constexpr int KT = BN * ROW;        // bytes of a K (or V) tile
     static constexpr int TILE = 2 * KT;
 };
@@ -58,11 +59,15 @@ struct PipeCfg {
 // CAP: soft cap (scores are capped and in log2 units once their maximum is taken)
 template <int DT, int HD, int RBLK, bool PAGED, bool ROT, bool CAP>
 __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
-    using C = PipeCfg<HD, RBLK>;
+    constexpr bool F8 = DT == DT_FP8;
+    constexpr int EB = F8 ? 1 : 2;
+    static_assert(!(F8 && ROT), "no rotary with FP8");
+    using C = PipeCfg<HD, RBLK, EB>;
     constexpr int RB = C::RB, BM = C::BM, BN = C::BN, NH = C::NH, KS = C::KS, DB = C::DB, CH = C::CH, ROW = C::ROW,
                   KT = C::KT, TILE = C::TILE, NE = 16 * RB;
     // slots: S products, then the P.V products of the first and the last 16 keys
-    constexpr int SS = KS * RB, SP = DB * RB;
+    constexpr int QS = KS * 2 / EB;  // S products per row block: an FP8 read is two bf16 operands
+    constexpr int SS = QS * RB, SP = DB * RB;
     static_assert(KT == 4 * 4 * 1024, "four loads of four waves bring a tile");
     __shared__ __attribute__((aligned(256))) char s_t[NBUF * TILE];
     __shared__ int s_pref[kMaxBatchLds + 1], s_ord[kOrdered];
@@ -74,15 +79,21 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
     else build_schedule<BM, C::BN, NT, 4>(a, s_pref, s_red, total, chunk_auto);
 
     const unsigned lds0 = lds_addr(s_t);
-    const unsigned rowa = lds0 + col * ROW + (slot_of<HD>(col, hi) << 4);  // chunk 2s + hi: ^ (s << 5)
+    const unsigned rowa = lds0 + col * ROW + (slot_of<ROW>(col, hi) << 4);  // chunk 2s + hi: ^ (s << 5)
     const int tr_r = 4 * hi + ((lane & 15) >> 2), tr_c = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-    const unsigned tra = lds0 + KT + tr_r * ROW + (slot_of<HD>(tr_r, tr_c) << 4) + (lane & 1) * 8;  // dim block db: ^ (db << 6)
+    // dim block db: ^ (db << 6). FP8: a group of 16 lanes reads 8 rows of one chunk,
+    // those of a whole operand: rows 4hi .. + 3 and 8 + 4hi .. + 3; db: ^ (db << 5)
+    const int tr8_r = 4 * hi + ((lane >> 1) & 3) + 8 * ((lane >> 3) & 1);
+    const unsigned tra = lds0 + KT + (lane & 1) * 8 +
+                         (F8 ? tr8_r * ROW + (slot_of<ROW>(tr8_r, (lane >> 4) & 1) << 4)
+                             : tr_r * ROW + (slot_of<ROW>(tr_r, tr_c) << 4));
 
-    const uint16_t* qp = static_cast<const uint16_t*>(a.q);
+    const char* qp = static_cast<const char*>(a.q);
     uint16_t* op = static_cast<uint16_t*>(a.out);
-    const float cs = CAP ? 1.f : a.scale_log2;
+    float cs = CAP ? 1.f : a.scale_log2;  // (FP8: times the item's descales)
     // cap * tanh(scale s / cap) in log2 units = c1 - 2 c1 / (2^(c0 s) + 1)
-    [[maybe_unused]] const float c0 = CAP ? 2.f * a.scale_log2 / a.softcap : 0.f, c1 = a.softcap * kLog2e;
+    [[maybe_unused]] float c0 = CAP ? 2.f * a.scale_log2 / a.softcap : 0.f;
+    [[maybe_unused]] const float c1 = a.softcap * kLog2e;
 
     for (int k = 0; k * (int)gridDim.x < total; ++k) {
         const int w = k * (int)gridDim.x + ((k & 1) ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x);
@@ -125,17 +136,17 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 
         // ---- K / V tiles straight into LDS -------------------------------------------------
         const int kvh = hk / a.kvdiv;
-        const char* kb = static_cast<const char*>(a.k) + 2 * (int64_t)kvh * a.k_sh;
-        const char* vb = static_cast<const char*>(a.v) + 2 * (int64_t)kvh * a.v_sh;
+        const char* kb = static_cast<const char*>(a.k) + EB * (int64_t)kvh * a.k_sh;
+        const char* vb = static_cast<const char*>(a.v) + EB * (int64_t)kvh * a.v_sh;
         [[maybe_unused]] const int* btrow = nullptr;
         if constexpr (PAGED) {
             btrow = a.block_table + (int64_t)crow * a.bt_stride;
         } else if (a.cu_seqlens_k) {
-            kb += 2 * ((int64_t)a.cu_seqlens_k[b] + base) * a.k_si;
-            vb += 2 * ((int64_t)a.cu_seqlens_k[b] + base) * a.v_si;
+            kb += EB * ((int64_t)a.cu_seqlens_k[b] + base) * a.k_si;
+            vb += EB * ((int64_t)a.cu_seqlens_k[b] + base) * a.v_si;
         } else {
-            kb += 2 * ((int64_t)crow * a.k_sb + (int64_t)(bi.lp + base) * a.k_si);
-            vb += 2 * ((int64_t)crow * a.v_sb + (int64_t)(bi.lp + base) * a.v_si);
+            kb += EB * ((int64_t)crow * a.k_sb + (int64_t)(bi.lp + base) * a.k_si);
+            vb += EB * ((int64_t)crow * a.v_sb + (int64_t)(bi.lp + base) * a.v_si);
         }
         // Load u of the wave brings rows RPL * (4 wave + u) .., lane l chunk slot
         // l % CH of row l / CH (the swizzle is in the address read). Rows past
@@ -144,12 +155,12 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int r = C::RPL * (4 * wave + u) + lane / CH;
-            const int c = min(slot_of<HD>(r, lane % CH), (a.hd >> 3) - 1);  // chunks past the head dim: q is 0 there
+            const int c = min(slot_of<ROW>(r, lane % CH), EB * a.hd / 16 - 1);  // chunks past the head dim: q is 0 there
             const int rl = min(r, k_hi - 1 - base - (ntiles - 1) * BN);
-            ko[0][u] = 2u * (unsigned)(r * (int)a.k_si + c * 8) + (3 - u) * 1024;
-            vo[0][u] = 2u * (unsigned)(r * (int)a.v_si + c * 8) + (3 - u) * 1024;
-            ko[1][u] = 2u * (unsigned)(rl * (int)a.k_si + c * 8) + (3 - u) * 1024;
-            vo[1][u] = 2u * (unsigned)(rl * (int)a.v_si + c * 8) + (3 - u) * 1024;
+            ko[0][u] = (unsigned)(EB * r * (int)a.k_si + c * 16) + (3 - u) * 1024;
+            vo[0][u] = (unsigned)(EB * r * (int)a.v_si + c * 16) + (3 - u) * 1024;
+            ko[1][u] = (unsigned)(EB * rl * (int)a.k_si + c * 16) + (3 - u) * 1024;
+            vo[1][u] = (unsigned)(EB * rl * (int)a.v_si + c * 16) + (3 - u) * 1024;
         }
         // Tiles are asked for in order; tiles past the end are the last one again.
         // Paged: page, first row in it and (read one tile early) block of the next.
@@ -185,13 +196,13 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
                 v4[u] = last ? vo[1][u] : vo[0][u];
                 if constexpr (decltype(first)::value && PAGED) {  // rows before the item's first key load that key
                     const unsigned up = (unsigned)max(0, k_lo - base - (C::RPL * (4 * wave + u) + lane / CH));
-                    k4[u] += 2u * up * (unsigned)a.k_si;
-                    v4[u] += 2u * up * (unsigned)a.v_si;
+                    k4[u] += EB * up * (unsigned)a.k_si;
+                    v4[u] += EB * up * (unsigned)a.v_si;
                 }
             }
             const unsigned wb = lds0 + TILE * buf + wave * 4096;
-            dma16x4(wb, kb + 2 * ok - 3072, k4);
-            dma16x4(wb + KT, vb + 2 * ov - 3072, v4);
+            dma16x4(wb, kb + EB * ok - 3072, k4);
+            dma16x4(wb + KT, vb + EB * ov - 3072, v4);
         };
         if (ntiles > 0) {
             load_tile(0, 0, std::true_type{});
@@ -199,9 +210,23 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             load_tile(2, 2, std::false_type{});
         }
 
+        [[maybe_unused]] float sc_v = 1.f;
+        [[maybe_unused]] uint32_t flip = 0;
+        if constexpr (F8) {
+            const float qk = descale_at(a.qd, a.qd_sb, a.qd_sh, b, kvh) * descale_at(a.kd, a.kd_sb, a.kd_sh, b, kvh);
+            sc_v = descale_at(a.vd, a.vd_sb, a.vd_sh, b, kvh);
+            if constexpr (CAP) {
+                c0 = 2.f * a.scale_log2 * qk / a.softcap;
+            } else {
+                // a negative factor goes to the signs of q; 0 must not meet the masks' infinity
+                cs = a.scale_log2 * qk;
+                flip = cs < 0.f ? 0x80008000u : 0u;
+                cs = cs == 0.f ? 1e-30f : fabsf(cs);
+            }
+        }
         // ---- q as B operands: lane holds row col, chunks 2s + hi -------------------------------
         const int wrow0 = tile_row0 + wave * RB * 32;
-        u32x4 qreg[RB][KS];
+            u32x4 qreg[RB][QS];
         int rlo[RB], rhi[RB];  // the row's visible keys, as offsets from the item's first tile
         [[maybe_unused]] int qi[RB];
         [[maybe_unused]] const uint16_t* qrows[RB];
@@ -212,16 +237,22 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             const int i = ok ? r / g : 0, h = hk * g + (ok ? r % g : 0);
             rlo[rb] = max(k_lo, key_lo(i + diag0, a.wl, a.chunk)) - base - 4 * hi;
             rhi[rb] = min(k_hi - 1, key_hi(i + diag0, a.wr, a.chunk)) - base - 4 * hi;
-            const uint16_t* qrow = a.cu_seqlens_q
-                                       ? qp + ((int64_t)a.cu_seqlens_q[b] + i) * a.q_si + (int64_t)h * a.q_sh
-                                       : qp + (int64_t)b * a.q_sb + (int64_t)i * a.q_si + (int64_t)h * a.q_sh;
+            const char* qrow = qp + EB * ((a.cu_seqlens_q ? ((int64_t)a.cu_seqlens_q[b] + i) * a.q_si
+                                                          : (int64_t)b * a.q_sb + (int64_t)i * a.q_si) + (int64_t)h * a.q_sh);
 #pragma unroll
-            for (int s = 0; s < KS; ++s)
-                qreg[rb][s] = ok && (2 * s + hi) * 8 < a.hd ? *reinterpret_cast<const u32x4*>(qrow + (2 * s + hi) * 8)
-                                                            : u32x4{0u, 0u, 0u, 0u};
+            for (int s = 0; s < KS; ++s) {
+                const int c = 2 * s + hi;
+                const u32x4 x = ok && c * 16 < EB * a.hd ? *reinterpret_cast<const u32x4*>(qrow + c * 16) : u32x4{0u, 0u, 0u, 0u};
+                if constexpr (F8) {
+                    qreg[rb][2 * s] = fp8x8_to_bf16(u32x2{x[0], x[1]}) ^ flip;
+                    qreg[rb][2 * s + 1] = fp8x8_to_bf16(u32x2{x[2], x[3]}) ^ flip;
+                } else {
+                    qreg[rb][s] = x;
+                }
+            }
             if constexpr (ROT) {
                 qi[rb] = i;
-                qrows[rb] = qrow;
+                qrows[rb] = reinterpret_cast<const uint16_t*>(qrow);
             }
         }
         if constexpr (ROT) {
@@ -254,7 +285,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int s = 0; s < KS; ++s) asm volatile("" : "+a"(qreg[rb][s]));
+            for (int s = 0; s < QS; ++s) asm volatile("" : "+a"(qreg[rb][s]));
 
         f32x16 o[RB][DB];
         float m[RB], l[RB];
@@ -275,14 +306,15 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
         for (int s = 0; s < KS; ++s) ra[s] = rowa ^ (s << 5);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            ta[db] = tra ^ (db << 6);
-            tb[db] = (tra ^ (db << 6) ^ 32) + 8 * ROW;
+            ta[db] = tra ^ (db << (F8 ? 5 : 6));
+            tb[db] = (tra ^ (db << 6) ^ 32) + 8 * ROW;  // (FP8: one read)
         }
         auto move_on = [&](unsigned& x, unsigned by) {
             x += by;
             asm volatile("" : "+v"(x));
         };
-        u32x4 kop[KS], vop[2 * DB];
+        u32x4 kop[KS];
+        std::conditional_t<F8, u32x2, u32x4> vop[2 * DB];
         auto read_rows = [&](int h, int s) {  // steps s and s + 1
             kop[s] = row_read(ra[s] + h * 32 * ROW);
             kop[s + 1] = row_read(ra[s + 1] + h * 32 * ROW);
@@ -291,7 +323,8 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
             for (int i = x; i < x + 2; ++i) {
                 const int o_ = (h * 32 + i / DB * 16) * ROW;
-                vop[i] = tr_read(ta[i % DB] + o_, tb[i % DB] + o_);
+                if constexpr (F8) vop[i] = tr8_read(ta[i % DB] + o_);
+                else vop[i] = tr_read(ta[i % DB] + o_, tb[i % DB] + o_);
             }
         };
 
@@ -321,6 +354,15 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
                         for (int i = 0; i < 16; ++i) o[rb][db][i] *= alpha;
                     }
                 }
+            }
+        };
+        // operand d of the reads s and s + 1
+        auto k_operand = [&](const u32x4 (&x)[KS], int s, int d) -> u32x4 {
+            if constexpr (F8) {
+                const u32x4 r = x[s + d / 2];
+                return fp8x8_to_bf16(d & 1 ? u32x2{r[2], r[3]} : u32x2{r[0], r[1]});
+            } else {
+                return x[s + d];
             }
         };
         const f32x16 zero = {};
@@ -362,24 +404,29 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
 #pragma unroll
             for (int s = 0; s < KS; s += 2) {
 #pragma unroll
-                for (int d = 1; d >= 0; --d)
+                for (int d = 4 / EB - 1; d >= 0; --d) {
+                    const u32x4 ka = k_operand(kop, s, d);
 #pragma unroll
                     for (int rb = 0; rb < RB; ++rb) {
-                        n_[rb] = mfma32<DT>(kop[s + d], qreg[rb][s + d], s == 0 && d == 1 ? zero : n_[rb]);
-                        if (d == 1 && rb == 0) {
+                        n_[rb] = mfma32<DT>(ka, qreg[rb][s * 2 / EB + d], s == 0 && d == 4 / EB - 1 ? zero : n_[rb]);
+                        if (d == 4 / EB - 1 && rb == 0) {
                             if (s + 2 < KS) read_rows(A, s + 2);
                             else read_tr(B, 0);
                         }
                         next();
                     }
+                }
             }
 #pragma unroll
             for (int x = 0; x < 2 * DB; x += 2) {
 #pragma unroll
-                for (int d = 1; d >= 0; --d)
+                for (int d = 1; d >= 0; --d) {
+                    u32x4 vt;
+                    if constexpr (F8) vt = fp8x8_to_bf16(vop[x + d]);
+                    else vt = vop[x + d];
 #pragma unroll
                     for (int rb = 0; rb < RB; ++rb) {
-                        o[rb][(x + d) % DB] = mfma32<DT>(vop[x + d], pk[rb][(x + d) / DB], o[rb][(x + d) % DB]);
+                        o[rb][(x + d) % DB] = mfma32<DT>(vt, pk[rb][(x + d) / DB], o[rb][(x + d) % DB]);
                         if (d == 1 && rb == 0) {
                             if (x + 2 < 2 * DB) read_tr(B, x + 2);
                             else ahead();
@@ -387,6 +434,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
                         more(x * RB + (1 - d) * RB + rb);
                         next();
                     }
+                }
             }
         };
 
@@ -401,7 +449,10 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             for (int rb = 0; rb < RB; ++rb) {
                 s0[rb] = zero;
 #pragma unroll
-                for (int s = 0; s < KS; ++s) s0[rb] = mfma32<DT>(kop[s], qreg[rb][s], s0[rb]);
+                for (int s = 0; s < KS; s += 2)
+#pragma unroll
+                    for (int d = 0; d < 4 / EB; ++d)
+                        s0[rb] = mfma32<DT>(k_operand(kop, s, d), qreg[rb][s * 2 / EB + d], s0[rb]);
             }
 #pragma unroll
             for (int e = 0; e < NE; ++e) {
@@ -503,7 +554,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             const int r = wrow0 + rb * 32 + col;
             const float lrow = l[rb] + __shfl_xor(l[rb], 32);
             const bool nonempty = lrow > 0.f;
-            const float inv = nonempty ? 1.f / lrow : 0.f;
+            const float inv = nonempty ? (F8 ? sc_v / lrow : 1.f / lrow) : 0.f;
             const float lse = nonempty ? (m[rb] + fast_log2(lrow)) * kLn2 : (final_out ? INFINITY : -INFINITY);
             if (r >= bi.rows) continue;
             const int i = r / g, h = hk * g + r % g;
@@ -546,6 +597,9 @@ void launch_t(const FwdArgs& a, int grid, hipStream_t stream) {
     if (a.softcap > 0.f) {
         if (a.block_table) go(fa_prefill_pipe_kernel<DT, HD, RB, true, false, true>);
         else go(fa_prefill_pipe_kernel<DT, HD, RB, false, false, true>);
+    } else if constexpr (DT == DT_FP8) {
+        if (a.block_table) go(fa_prefill_pipe_kernel<DT, HD, RB, true, false, false>);
+        else go(fa_prefill_pipe_kernel<DT, HD, RB, false, false, false>);
     } else if (a.block_table) {
         if (a.rot_cos) go(fa_prefill_pipe_kernel<DT, HD, RB, true, true, false>);
         else go(fa_prefill_pipe_kernel<DT, HD, RB, true, false, false>);

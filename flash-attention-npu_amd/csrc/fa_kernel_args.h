@@ -92,14 +92,16 @@ struct FwdArgs {
 };
 
 // Which prefill calls run on the pipelined kernel (fa_fwd_pipe.h); the others
-// keep the kernel of fa_fwd.hip. d: kernel head dim; dtype 0 / 1: fp16 / bf16.
+// keep the kernel of fa_fwd.hip. d: kernel head dim; dtype 0 / 1 / 3: fp16 / bf16 /
+// e4m3 (at head dim 128).
 // The rows of a tile (16 KB) have 32-bit byte offsets, and a paged tile lies in
 // one page.
 inline bool prefill_pipe_takes(int dtype, int d, float scale, float softcap, bool alibi, bool rotary, int64_t k_si,
                                int64_t v_si, bool paged, int page) {
     auto fits = [](int64_t si) { return si >= 0 && si < (1 << 22); };
-    return (dtype == 0 || dtype == 1) && scale > 0.f && !alibi && !(softcap > 0.f && rotary) && fits(k_si) &&
-           fits(v_si) && (!paged || page % (8192 / d) == 0);
+    const bool f8 = dtype == 3;
+    return (dtype == 0 || dtype == 1 || (f8 && d == 128)) && scale > 0.f && !alibi && !(softcap > 0.f && rotary) &&
+           fits(k_si) && fits(v_si) && (!paged || page % ((f8 ? 16384 : 8192) / d) == 0);
 }
 
 // Backward (dense / varlen). Row layouts as in FwdArgs; lse and dsum share

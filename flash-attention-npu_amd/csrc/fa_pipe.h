@@ -39,6 +39,13 @@ __device__ __forceinline__ u32x4 tr_read(unsigned lo, unsigned hi) {
     const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(size_t)hi));
     return u32x4{a[0], a[1], b[0], b[1]};
 }
+// 8 rows of one byte column: of 16 lanes, lane i gives the address of 8 bytes
+// (half i & 1 of 16 columns) of row i >> 1 and gets column i
+__device__ __forceinline__ u32x2 tr8_read(unsigned a) {
+    typedef int i32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(size_t)a));
+}
 __device__ __forceinline__ u32x4 row_read(unsigned a) {
     return *(const __attribute__((address_space(3))) u32x4*)(size_t)a;
 }

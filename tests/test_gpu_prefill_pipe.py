@@ -124,3 +124,54 @@ def test_ragged(causal, d):
                            cu_seqlens_k=cu, max_seqlen_q=700, nthreads=NT)
     assert_close_out(out, ro, torch.bfloat16)
     assert_close_lse(lse, rl)
+
+
+@pytest.mark.parametrize("b,sq,sk", [(1, 17, 40), (1, 128, 128), (2, 257, 129), (3, 300, 1100), (16, 520, 513)])
+@pytest.mark.parametrize("d", [80, 128])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_fp8(b, sq, sk, d, softcap):
+    """e4m3 inputs with descales of either sign and zero, row tiles of both kinds."""
+    import flash_attn_npu_v3
+    print(f"case pipe fp8 B{b} {sq}x{sk} D{d} softcap={softcap}", flush=True)
+    f8 = torch.float8_e4m3fn
+    q, k, v = inputs(sq, torch.bfloat16, (b, sq, 8, d), (b, sk, 2, d), (b, sk, 2, d))
+    q, k, v = q.to(f8), k.to(f8), v.to(f8)
+    g = torch.Generator().manual_seed(1)
+    qd, kd, vd = (0.5 + torch.rand((b, 2), generator=g) for _ in range(3))
+    qd[0, 0], kd[b - 1, 1] = -1.25, 0.0
+    out, lse = flash_attn_npu_v3.flash_attn_func(q.cuda(), k.cuda(), v.cuda(), causal=True, softcap=softcap,
+                                                 q_descale=qd.cuda(), k_descale=kd.cuda(), v_descale=vd.cuda(),
+                                                 return_attn_probs=True)
+    by = lambda x: x.view(torch.uint8).numpy()
+    ro, rl = orc.attention_fp8(by(q), by(k), by(v), scale=d ** -0.5, q_descale=qd.numpy(), k_descale=kd.numpy(),
+                               v_descale=vd.numpy(), causal=True, softcap=softcap, nthreads=NT)
+    err = (out.float().cpu() - torch.from_numpy(ro)).abs()
+    # 1e-2 + one bf16 ulp of the reference, as for bf16 inputs (outputs here reach v_descale x 4)
+    assert bool((err <= 1e-2 + 2.0 ** -7 * torch.from_numpy(ro).abs()).all()), float(err.max())
+    assert_close_lse(lse, rl)
+
+
+@pytest.mark.parametrize("page", [0, 64, 128, 256])
+def test_fp8_kvcache(page):
+    """A cache of e4m3 rows, paged where a tile lies in one page and where it does not, and a split of the keys."""
+    import flash_attn_npu_v3
+    f8 = torch.float8_e4m3fn
+    B, Sq, Hk, D, lens = 2, 70, 2, 128, [1500, 333]
+    q, k, v = inputs(page, torch.bfloat16, (B, Sq, 8, D), (B, 1536, Hk, D), (B, 1536, Hk, D))
+    q, k, v = q.to(f8), k.to(f8), v.to(f8)
+    by = lambda x: x.view(torch.uint8).numpy()
+    ro, rl = orc.attention_fp8(by(q), by(k), by(v), scale=D ** -0.5, causal=True, nthreads=NT,
+                               seqlens_k=np.array(lens, np.int32))
+    more = {}
+    kc, vc = k.cuda(), v.cuda()
+    if page:
+        n = 1536 // page
+        more["page_table"] = torch.arange(B * n, dtype=torch.int32).view(B, n).cuda()
+        kc, vc = (x.reshape(B * n, page, Hk, D) for x in (kc, vc))
+    for ns in (0, 3):
+        out, lse, _, _ = flash_attn_npu_v3.flash_attn_with_kvcache(
+            q.cuda(), kc, vc, cache_seqlens=torch.tensor(lens, dtype=torch.int32).cuda(), causal=True, num_splits=ns,
+            return_softmax_lse=True, **more)
+        err = (out.float().cpu() - torch.from_numpy(ro)).abs()
+        assert bool((err <= 1e-2 + 2.0 ** -7 * torch.from_numpy(ro).abs()).all()), float(err.max())
+        assert_close_lse(lse, rl)
