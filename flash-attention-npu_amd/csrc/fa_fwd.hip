@@ -1,6 +1,9 @@
 // fa_fwd.hip -- FlashAttention forward (prefill / chunked prefill / dense /
 // varlen) for gfx950 (MI355X), the split-KV merge, and the standalone
-// log-sum-exp combine.
+// log-sum-exp combine. Most calls run on the pipelined kernel (fa_fwd_pipe.h,
+// chosen by prefill_pipe_takes); the one here keeps those with ALiBi, a soft cap
+// together with rotary, a non-positive scale, pages that a 16 KB tile does not
+// divide, row strides of 2^22 elements and more, and FP8 outside head dims 65..128.
 //
 // Reference behaviour being reproduced (paths relative to the reference repo):
 //   SplitFuse::FAInfer / runMainLoop  csrc/arch22/flash_attn_npu_v2/mha_fwd_kvcache.cpp:436-966
@@ -15,7 +18,8 @@
 //   * S^T = K.Q^T with 16x16x32 MFMA: the accumulator then holds, per lane, one
 //     query row and 8 keys, which is exactly the packed P^T operand of
 //     O^T = V^T.P^T. The head dimension of Q/K is permuted (lane group G takes
-//     dims G*D/4 .. +D/4) so every lane reads contiguous 16-byte chunks.
+//     16-byte chunk 4s + G in step s): every lane reads whole chunks, and the
+//     K reads have no bank conflicts.
 //   * One workgroup = 8 waves x 32 rows (two waves per SIMD); a wave reuses
 //     each K/V operand it reads from LDS for its 2 row blocks of 16. The
 //     256-VGPR budget of two waves per SIMD is what bounds the row blocks.
