@@ -74,6 +74,14 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
     __shared__ long long s_red[8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hi = lane >> 5;
+    // K chunks past the head dim are 0 and stay so (no load writes them): q is 0
+    // there, but another chunk's infinity times 0 is not. e4m3 has no infinity.
+    if (!F8 && a.hd < HD) {
+#pragma unroll
+        for (int x = 0; x < NBUF; ++x)
+            for (int at = tid * 16; at < KT; at += NT * 16) row_write(lds_addr(s_t) + x * TILE + at, u32x4{0u, 0u, 0u, 0u});
+        __syncthreads();
+    }
     int total, chunk_auto = 0;
     if (ordered(a)) total = ordered_schedule<BM>(a, s_pref, s_ord);
     else build_schedule<BM, C::BN, NT, 4>(a, s_pref, s_red, total, chunk_auto);
@@ -152,10 +160,12 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
         // l % CH of row l / CH (the swizzle is in the address read). Rows past
         // the last key of the item load that key: second set, for the last tile.
         unsigned ko[2][4], vo[2][4];
+        [[maybe_unused]] uint64_t in_hd[4];  // K load u: lanes whose chunk lies in the head dim
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int r = C::RPL * (4 * wave + u) + lane / CH;
-            const int c = min(slot_of<ROW>(r, lane % CH), EB * a.hd / 16 - 1);  // chunks past the head dim: q is 0 there
+            const int c = min(slot_of<ROW>(r, lane % CH), EB * a.hd / 16 - 1);  // V: what is past the head dim is not written out
+            in_hd[u] = __ballot(slot_of<ROW>(r, lane % CH) < EB * a.hd / 16);
             const int rl = min(r, k_hi - 1 - base - (ntiles - 1) * BN);
             ko[0][u] = (unsigned)(EB * r * (int)a.k_si + c * 16) + (3 - u) * 1024;
             vo[0][u] = (unsigned)(EB * r * (int)a.v_si + c * 16) + (3 - u) * 1024;
@@ -201,7 +211,8 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
                 }
             }
             const unsigned wb = lds0 + TILE * buf + wave * 4096;
-            dma16x4(wb, kb + EB * ok - 3072, k4);
+            if constexpr (F8) dma16x4(wb, kb + EB * ok - 3072, k4);
+            else dma16x4(wb, kb + EB * ok - 3072, k4, in_hd);
             dma16x4(wb + KT, vb + EB * ov - 3072, v4);
         };
         if (ntiles > 0) {

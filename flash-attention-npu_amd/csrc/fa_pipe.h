@@ -75,6 +75,22 @@ __device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const un
         "global_load_lds_dwordx4 %5, %1 offset:3072" ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3])
         : "memory");
 }
+// The same by the lanes of mask[u] in load u; the LDS bytes of the others stay
+__device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const unsigned (&off)[4], const uint64_t (&mask)[4]) {
+    base = uniform(base);
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    uint64_t all;
+    asm volatile(
+        "s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\t"
+        "s_mov_b64 exec, %7\n\tglobal_load_lds_dwordx4 %3, %2\n\t"
+        "s_mov_b64 exec, %8\n\tglobal_load_lds_dwordx4 %4, %2 offset:1024\n\t"
+        "s_mov_b64 exec, %9\n\tglobal_load_lds_dwordx4 %5, %2 offset:2048\n\t"
+        "s_mov_b64 exec, %10\n\tglobal_load_lds_dwordx4 %6, %2 offset:3072\n\t"
+        "s_mov_b64 exec, %0"
+        : "=&s"(all)
+        : "s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(mask[0]), "s"(mask[1]), "s"(mask[2]), "s"(mask[3])
+        : "memory");
+}
 __device__ __forceinline__ void dma4(unsigned lds, const char* base, unsigned off) {
     base = uniform(base);
     lds = __builtin_amdgcn_readfirstlane(lds);

@@ -48,6 +48,22 @@ def test_head_dims(b, sq, d):
     dense(torch.float16, b, 4, 4, sq, 130, d, seed=d)
 
 
+@pytest.mark.parametrize("d", [40, 64, 72, 120, 128, 160])
+def test_infinite_key(d):
+    """A key of -inf in the last dimension, against positive q: weight 0, nothing else touched."""
+    import flash_attn_npu_v2
+    print(f"case pipe -inf key D{d}", flush=True)
+    q, k, v = inputs(d, torch.bfloat16, (2, 150, 4, d), (2, 200, 2, d), (2, 200, 2, d))
+    q[..., -1] = 1.0
+    k[:, 77, :, -1] = -float("inf")
+    out, lse, _ = flash_attn_npu_v2.flash_attn_func(q.cuda(), k.cuda(), v.cuda(), return_attn_probs=True)
+    keep = [j for j in range(200) if j != 77]
+    ro, rl = orc.attention(bits(q), bits(k[:, keep].contiguous()), bits(v[:, keep].contiguous()), dtype=odt(torch.bfloat16),
+                           scale=d ** -0.5, nthreads=NT)
+    assert_close_out(out, ro, torch.bfloat16)
+    assert_close_lse(lse, rl)
+
+
 @pytest.mark.parametrize("window", [(0, 0), (63, 0), (64, 3), (100, -1), (-1, 70)])
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_windows(window, d):
