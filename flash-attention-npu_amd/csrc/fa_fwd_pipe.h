@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
         }
         // ---- q as B operands: lane holds row col, chunks 2s + hi -------------------------------
         const int wrow0 = tile_row0 + wave * RB * 32;
-            u32x4 qreg[RB][QS];
+        u32x4 qreg[RB][QS];
         int rlo[RB], rhi[RB];  // the row's visible keys, as offsets from the item's first tile
         [[maybe_unused]] int qi[RB];
         [[maybe_unused]] const uint16_t* qrows[RB];
