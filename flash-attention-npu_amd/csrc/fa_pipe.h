@@ -63,17 +63,20 @@ __device__ __forceinline__ const char* uniform(const char* p) {
 // instruction's offset moves both addresses, so off[u] holds (3 - u) KB more
 // and `base` is 3 KB less. In assembly, because the compiler would wait for
 // every such load before any LDS read; wait_loads<N> waits until all but the
-// wave's last N are there.
+// wave's last N are there. Nor does it put wait states inside the block: five
+// instructions' worth lie between the readfirstlanes of the address and the first
+// load (gfx9's distance from a vector write of a scalar register to a memory
+// instruction that reads it), the write of m0 among them.
 __device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const unsigned (&off)[4]) {
     base = uniform(base);
     lds = __builtin_amdgcn_readfirstlane(lds);
     asm volatile(
-        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "s_mov_b32 m0, %0\n\ts_nop 3\n\t"
         "global_load_lds_dwordx4 %2, %1\n\t"
         "global_load_lds_dwordx4 %3, %1 offset:1024\n\t"
         "global_load_lds_dwordx4 %4, %1 offset:2048\n\t"
         "global_load_lds_dwordx4 %5, %1 offset:3072" ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3])
-        : "memory");
+        : "memory", "m0");
 }
 // The same by the lanes of mask[u] in load u; the LDS bytes of the others stay
 __device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const unsigned (&off)[4], const uint64_t (&mask)[4]) {
@@ -81,7 +84,7 @@ __device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const un
     lds = __builtin_amdgcn_readfirstlane(lds);
     uint64_t all;
     asm volatile(
-        "s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\t"
+        "s_mov_b32 m0, %1\n\ts_mov_b64 %0, exec\n\ts_nop 1\n\t"
         "s_mov_b64 exec, %7\n\tglobal_load_lds_dwordx4 %3, %2\n\t"
         "s_mov_b64 exec, %8\n\tglobal_load_lds_dwordx4 %4, %2 offset:1024\n\t"
         "s_mov_b64 exec, %9\n\tglobal_load_lds_dwordx4 %5, %2 offset:2048\n\t"
@@ -89,12 +92,12 @@ __device__ __forceinline__ void dma16x4(unsigned lds, const char* base, const un
         "s_mov_b64 exec, %0"
         : "=&s"(all)
         : "s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(mask[0]), "s"(mask[1]), "s"(mask[2]), "s"(mask[3])
-        : "memory");
+        : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(unsigned lds, const char* base, unsigned off) {
     base = uniform(base);
     lds = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %2, %1" ::"s"(lds), "s"(base), "v"(off) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %2, %1" ::"s"(lds), "s"(base), "v"(off) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {
