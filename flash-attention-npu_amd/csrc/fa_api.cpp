@@ -100,6 +100,10 @@ struct Plan {
     size_t off_sched, off_plse, off_po, off_qrot, total;
 };
 
+// A window bound for the kernels (-1: none). They add it to positions in 32 bits:
+// no sequence is longer than 2^30, so a wider window hides nothing either.
+int window_bound(int32_t w) { return w < 0 ? -1 : std::min(w, 1 << 30); }
+
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 fa_status_t validate(const fa_fwd_params* p, int kind) {
@@ -558,8 +562,7 @@ fa_status_t run_forward_ws(const fa_fwd_params* p, int kind, void* stream_v, voi
         }
         // window normalisation (flash_api.cpp:483-494): the seqlen-dependent rules
         // leave the mask unchanged, causal forces the right edge to the diagonal
-        int wl = p->window_size_left < 0 ? -1 : p->window_size_left;
-        int wr = p->window_size_right < 0 ? -1 : p->window_size_right;
+        int wl = window_bound(p->window_size_left), wr = window_bound(p->window_size_right);
         if (p->is_causal) wr = 0;
         a.wl = wl;
         a.wr = wr;
@@ -728,8 +731,7 @@ fa_status_t run_backward(const fa_bwd_params* p, int kind, void* stream_v) {
         a.hd = p->headdim;
         a.total_q = p->total_q;
         // window normalisation as in the forward (flash_api.cpp:483-494)
-        int wl = p->window_size_left < 0 ? -1 : p->window_size_left;
-        int wr = p->window_size_right < 0 ? -1 : p->window_size_right;
+        int wl = window_bound(p->window_size_left), wr = window_bound(p->window_size_right);
         if (p->is_causal) wr = 0;
         a.wl = wl;
         a.wr = wr;

@@ -172,12 +172,14 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) dv[db][i] = dk[db][i] = 0.f;
 
-        // visible rows of this lane's key, relative to r_lo: [vlo, vhi); all keys of the wave: [flo, fhi)
-        const int vlo = a.wr >= 0 ? ((jl - diag0 - a.wr) << gs) - r_lo : -0x40000000;
-        const int vhi = a.wl >= 0 ? ((jl - diag0 + a.wl + 1) << gs) - r_lo : 0x40000000;
+        // visible rows of this lane's key, relative to r_lo: [vlo, vhi). In positions the
+        // bounds are cut to the sequence first: a window past it has no 32-bit row.
+        auto row_of = [&](int i) { return (min(max(i, 0), bb.sq) << gs) - r_lo; };
+        const int vlo = a.wr >= 0 ? row_of(jl - diag0 - a.wr) : -0x40000000;
+        const int vhi = a.wl >= 0 ? row_of(jl - diag0 + a.wl + 1) : 0x40000000;
         // tiles all of whose rows see all keys of the block: [t1, t2)
-        const int flo = a.wr >= 0 ? ((j0 + BK - 1 - diag0 - a.wr) << gs) - r_lo : 0;
-        const int fhi = a.wl >= 0 ? ((j0 - diag0 + a.wl + 1) << gs) - r_lo : nrows;
+        const int flo = a.wr >= 0 ? row_of(j0 + BK - 1 - diag0 - a.wr) : 0;
+        const int fhi = a.wl >= 0 ? row_of(j0 - diag0 + a.wl + 1) : nrows;
         const int t1 = min(ntiles, max(0, (flo + BQ - 1) / BQ));
         const int t2 = max(t1, a.wl >= 0 ? min(ntiles, max(0, fhi) / BQ) : ntiles);
 

@@ -33,6 +33,31 @@ def test_windows(window, dtype):
     run_dense(dtype, 1, 4, 1, 200, 210, 128, False, window=window, seed=7)
 
 
+@pytest.mark.parametrize("sides", [(1, None), (1, 0), (None, 1), (1, 1)], ids=["left", "left_causal", "right", "both"])
+@pytest.mark.parametrize("g", [1, 2, 4, 8, 64])
+@pytest.mark.parametrize("w", [1 << 25, 1 << 28, 10**9, 1 << 30, (1 << 31) - 1])
+def test_windows_past_the_sequence(w, g, sides):
+    """A window wider than the sequence hides nothing: the results of an
+    unbounded one bit for bit, also where the bound times the query heads per kv
+    head, or plus a position, is past 32 bits."""
+    import flash_attn_npu_v2
+    gen = torch.Generator().manual_seed(g)
+    for sq, sk in ((150, 150), (40, 200), (200, 40)):
+        q, do = (rand_inputs((1, sq, g, 128), torch.bfloat16, gen).cuda() for _ in range(2))
+        k, v = (rand_inputs((1, sk, 1, 128), torch.bfloat16, gen).cuda() for _ in range(2))
+
+        def run(window):
+            print(f"case wide window {window} g{g} {sq}x{sk}", flush=True)
+            parts = [x.detach().requires_grad_(True) for x in (q, k, v)]
+            out, lse, _ = flash_attn_npu_v2.flash_attn_func(*parts, window_size=window, return_attn_probs=True)
+            return (out, lse) + torch.autograd.grad(out, parts, do)
+
+        want = run(tuple(0 if x == 0 else -1 for x in sides))
+        got = run(tuple(-1 if x is None else x * w for x in sides))
+        for name, x, ref in zip(("out", "lse", "dq", "dk", "dv"), got, want):
+            assert torch.equal(x, ref), name
+
+
 @pytest.mark.parametrize("d", [72, 96, 120])
 def test_head_dims(d):
     run_dense(torch.float16, 2, 4, 2, 150, 140, d, True, seed=d, api="v3")

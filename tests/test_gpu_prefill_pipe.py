@@ -191,3 +191,20 @@ def test_fp8_kvcache(page):
         err = (out.float().cpu() - torch.from_numpy(ro)).abs()
         assert bool((err <= 1e-2 + 2.0 ** -7 * torch.from_numpy(ro).abs()).all()), float(err.max())
         assert_close_lse(lse, rl)
+
+
+@pytest.mark.parametrize("sq", [1, 4, 70])
+@pytest.mark.parametrize("page", [0, 64])
+def test_window_past_the_cache(sq, page):
+    """The widest windows there are hide nothing, in decode and prefill: the bounds are added to positions in 32 bits."""
+    import flash_attn_npu_v2
+    q, k, v = (x.cuda() for x in inputs(sq, torch.bfloat16, (2, sq, 8, 128), (2, 256, 2, 128), (2, 256, 2, 128)))
+    more = dict(cache_seqlens=torch.tensor([201, 33], dtype=torch.int32).cuda(), return_softmax_lse=True)
+    if page:
+        k, v = (x.reshape(-1, page, 2, 128) for x in (k, v))
+        more["block_table"] = torch.arange(512 // page, dtype=torch.int32).view(2, -1).cuda()
+    big = (1 << 31) - 1
+    for window, same in (((big, big), (-1, -1)), ((-1, big), (-1, -1)), ((big, 0), (-1, 0))):
+        print(f"case window {window} sq{sq} page{page}", flush=True)
+        got, want = (flash_attn_npu_v2.flash_attn_with_kvcache(q, k, v, window_size=w, **more) for w in (window, same))
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
