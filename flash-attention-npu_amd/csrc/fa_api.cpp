@@ -744,13 +744,21 @@ fa_status_t run_backward(const fa_bwd_params* p, int kind, void* stream_v) {
         // several items each (B4 S4096 H32/8 causal the same as with 2 x CUs
         // workgroups, B2 3-4 % faster), ragged ones on one workgroup per item
         // (up to 16 x CUs), counted from the rows in all and a part item per
-        // sequence; the keys are taken to be as many as the rows, as in self
-        // attention (the kernels walk on where there are more)
+        // sequence. How many keys there are in all is not known here: as many as
+        // rows where no sequence can have more keys than another has rows (self
+        // attention), though never fewer workgroups than fill the CUs; else
+        // as many as seqlen_k allows. The kernels walk on where there are more.
+        // Whole backward, us, counted from the rows always -> so: four times 16
+        // positions onto 8192 keys, H32/8 D128 783 -> 261 (D64 400 -> 140, H8/8
+        // D256 1454 -> 536); 2048 and 15 times 16 positions, each onto 2048 keys,
+        // H8/2 321 -> 262; 24 documents of 37 to 1024, causal, the same (476).
         const int cap = (p->cu_seqlens_q ? 16 : 1) * cu_count();
         auto packed = [&](int64_t items, int64_t rows, int block) {
             return p->cu_seqlens_q ? std::min(items, (rows / block + nb) * p->nheads_k) : items;
         };
-        const int grid_kv = (int)std::max<int64_t>(1, std::min<int64_t>(packed(gkv, p->total_q, fa::bwd_key_block(kd)), cap));
+        const int64_t kv_items = p->seqlen_k > p->seqlen_q ? gkv
+                                 : std::max<int64_t>(packed(gkv, p->total_q, fa::bwd_key_block(kd)), std::min<int64_t>(gkv, cu_count()));
+        const int grid_kv = (int)std::max<int64_t>(1, std::min<int64_t>(kv_items, cap));
         const int grid_q = (int)std::max<int64_t>(1, std::min<int64_t>(packed(gq, (int64_t)p->total_q * a.g, bm), cap));
         hipError_t e = fa::launch_bwd(a, p->dtype, kd, grid_kv, grid_q, static_cast<hipStream_t>(stream_v));
         if (e != hipSuccess) return fail(FA_EHIP, "backward launch failed: %s", hipGetErrorString(e));

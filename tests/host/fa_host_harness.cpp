@@ -39,6 +39,7 @@ struct Launch {
     const void* out;
     const float* lse;
     const int* seqlens;
+    int grid_kv, grid_q;  // backward
 };
 std::vector<Launch> g_launch;
 void rec(const char* k, int B, const void* q, const void* out, const float* lse, const int* sl) {
@@ -83,8 +84,10 @@ hipError_t launch_kv_prep(const KvPrepArgs& a, int, hipStream_t) {
     rec("kvprep", a.B, a.q, nullptr, nullptr, a.seqlens);
     return hipSuccess;
 }
-hipError_t launch_bwd(const BwdArgs& a, int, int, int, int, hipStream_t) {
+hipError_t launch_bwd(const BwdArgs& a, int, int, int grid_kv, int grid_q, hipStream_t) {
     rec("bwd", a.B, a.q, a.dq, a.lse, nullptr);
+    g_launch.back().grid_kv = grid_kv;
+    g_launch.back().grid_q = grid_q;
     return hipSuccess;
 }
 }  // namespace fa
@@ -241,6 +244,44 @@ int main() {
             cov += l.B;
         }
         EXPECT(cov == B, "bwd covered %d of %d", cov, B);
+    }
+
+    // a ragged backward's dK / dV workgroups follow the keys, also where there are few query rows: one per item
+    // of (sequence, kv head, key block), or at least as many as there are items or CUs
+    struct Ragged { int B, total_q, max_q, max_k, hk, d, want; };
+    const Ragged ragged[] = {
+        {4, 64, 16, 8192, 8, 128, 2048},   // 16 positions each onto 8192 keys
+        {1, 256, 256, 32768, 8, 128, 2048},
+        {2, 2, 1, 4096, 2, 256, 256},      // 64-key blocks
+        {2, 2064, 2048, 2048, 2, 128, 64}, // the short sequence of the rows may be the long one of the keys
+        {64, 2048, 32, 32, 1, 64, 64},
+    };
+    for (const Ragged& x : ragged) {
+        fa_bwd_params b;
+        memset(&b, 0, sizeof(b));
+        b.abi_version = FA_MI355X_ABI_VERSION;
+        b.dtype = FA_DTYPE_BF16;
+        b.batch = x.B;
+        b.seqlen_q = x.max_q;
+        b.seqlen_k = x.max_k;
+        b.total_q = x.total_q;
+        b.nheads = b.nheads_k = x.hk;
+        b.headdim = x.d;
+        b.q = b.k = b.v = b.out = b.dout = (const void*)0x100000;
+        b.dq = b.dk = b.dv = (void*)0x200000;
+        b.q_row_stride = b.out_row_stride = b.dout_row_stride = b.dq_row_stride = x.hk * x.d;
+        b.k_row_stride = b.v_row_stride = b.dk_row_stride = b.dv_row_stride = x.hk * x.d;
+        b.q_head_stride = b.k_head_stride = b.v_head_stride = b.out_head_stride = b.dout_head_stride = x.d;
+        b.dq_head_stride = b.dk_head_stride = b.dv_head_stride = x.d;
+        b.softmax_lse = (const float*)0x300000;
+        b.softmax_d = (float*)0x380000;
+        b.cu_seqlens_q = b.cu_seqlens_k = (const int32_t*)0x400000;
+        b.window_size_left = b.window_size_right = -1;
+        g_launch.clear();
+        EXPECT(fa_mha_varlen_bwd(&b, nullptr) == FA_OK && g_launch.size() == 1, "ragged bwd: %s", fa_last_error());
+        if (g_launch.size() == 1)
+            EXPECT(g_launch[0].grid_kv >= x.want, "ragged bwd B=%d q=%d k=%d: %d dK/dV workgroups for %d items", x.B,
+                   x.max_q, x.max_k, g_launch[0].grid_kv, x.want);
     }
 
     // invalid and extreme inputs must be refused (or accepted) without UB
