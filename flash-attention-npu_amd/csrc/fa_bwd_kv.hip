@@ -53,12 +53,19 @@ __device__ __forceinline__ u32x2 split3(float v) {
     return u32x2{h | (m << 16), l};
 }
 
-template <int DT>
+// PART: the head dim is below 128 (see fa_bwd_dq.hip)
+template <int DT, bool PART>
 __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
     __shared__ __attribute__((aligned(256))) uint16_t s_t[NBUF * TILE];
     __shared__ int s_pref[bw::kMaxBatch + 1], s_ord[kOrdered];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hi = lane >> 5;
+    if constexpr (PART) {  // q and dout chunks past the head dim are 0 and stay so, as K and V are there (barrier: in the prefix)
+#pragma unroll
+        for (int x = 0; x < NBUF; ++x)
+            for (int at = tid * 16; at < 4 * QT; at += NT * 16)
+                row_write(lds_addr(s_t) + x * 2 * TILE + at, u32x4{0u, 0u, 0u, 0u});
+    }
     const int total = bw_ordered_prefix<NT>(a, s_pref, s_ord, [&](int b) {
         const BwBatch bb = bw_batch(a, b);
         return a.Hk * ((bb.sk + BK - 1) / BK);
@@ -136,11 +143,12 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
         // l the 16 bytes of slot l % 16 of row l / 16 (the swizzle is in the
         // address read).
         unsigned qo[CPQ], dof[CPQ];
+        [[maybe_unused]] uint64_t in_hd[CPQ];  // load u: lanes whose chunk lies in the head dim
 #pragma unroll
         for (int u = 0; u < CPQ; ++u) {
             const int r = 16 * wave + 4 * u + (lane >> 4);
-            // chunks past the head dim load the last one (K and V are 0 there)
-            const int c = min(swz(r, lane & 15), (a.hd >> 3) - 1);
+            const int c = swz(r, lane & 15);
+            if constexpr (PART) in_hd[u] = __ballot(c < (a.hd >> 3));
             const int i = min(r >> gs, i_hi - i_lo), j = r & (g - 1);
             qo[u] = 2u * (unsigned)(i * (int)a.q_si + j * (int)a.q_sh + c * 8) + (3 - u) * 1024;
             dof[u] = 2u * (unsigned)(i * (int)a.do_si + j * (int)a.do_sh + c * 8) + (3 - u) * 1024;
@@ -149,8 +157,13 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
         auto load_tile = [&](int t, int buf) {  // tiles past the end: the last one
             const int64_t i = row0(min(t, ntiles - 1)) >> gs;
             const unsigned base = lds0 + 2 * TILE * buf, wb = base + wave * 16 * 2 * D;
-            dma16x4(wb, qt + i * q2 - 3072, qo);
-            dma16x4(wb + 2 * QT, dt + i * d2 - 3072, dof);
+            if constexpr (PART) {
+                dma16x4(wb, qt + i * q2 - 3072, qo, in_hd);
+                dma16x4(wb + 2 * QT, dt + i * d2 - 3072, dof, in_hd);
+            } else {
+                dma16x4(wb, qt + i * q2 - 3072, qo);
+                dma16x4(wb + 2 * QT, dt + i * d2 - 3072, dof);
+            }
             dma4(base + 4 * QT + 4 * ST + (wave & 1) * RAW, lt + 4 * i, so);
         };
         // this wave's row constants of tile t, once its loads are there
@@ -416,8 +429,10 @@ bool bwd_kv_takes(const BwdArgs& a) {
 }
 
 void launch_bwd_kv(const BwdArgs& a, int dtype, int grid, hipStream_t stream) {
-    if (dtype == DT_BF16) hipLaunchKernelGGL(fa_bwd_kv_kernel<DT_BF16>, dim3(grid), dim3(NT), 0, stream, a);
-    else hipLaunchKernelGGL(fa_bwd_kv_kernel<DT_FP16>, dim3(grid), dim3(NT), 0, stream, a);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, stream, a); };
+    const bool part = a.hd < D;
+    if (dtype == DT_BF16) part ? go(fa_bwd_kv_kernel<DT_BF16, true>) : go(fa_bwd_kv_kernel<DT_BF16, false>);
+    else part ? go(fa_bwd_kv_kernel<DT_FP16, true>) : go(fa_bwd_kv_kernel<DT_FP16, false>);
 }
 
 }  // namespace fa

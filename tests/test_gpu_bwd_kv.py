@@ -100,3 +100,30 @@ def test_dq_tiles(sq, sk, d, softcap):
 def test_dq_windows(d, window):
     run_dense(torch.float16, 1, 4, 1, 200, 210, d, False, window=window, softcap=15.0, seed=8)
     run_varlen(torch.bfloat16, 8, 2, [1, 200, 64, 0, 129], [130, 200, 1, 40, 128], d, False, window=window, seed=4)
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "do"])
+@pytest.mark.parametrize("d", [40, 72, 96, 120, 160])
+def test_infinity_below_the_kernel_head_dim(d, where):
+    """An infinity in the last dims of a row goes where it goes in the same
+    tensors with zeros up to the kernel's head dim (NaN for NaN), and no further:
+    what the kernels hold past the head dim is 0. The other tensors are
+    positive there, so that a key of -inf has weight 0 and its rows stay finite."""
+    import flash_attn_npu_v2
+    full = 64 if d <= 64 else 128 if d <= 128 else 256
+    g = torch.Generator().manual_seed(d)
+    x = {n: rand_inputs((1, 150, 2 if n in ("q", "do") else 1, d), torch.bfloat16, g) for n in ("q", "k", "v", "do")}
+    for t in x.values():
+        t[..., d - 3] = t[..., d - 3].abs() + 0.5
+    x[where][0, 70, 0, d - 3] = -float("inf")
+    print(f"case infinity in {where} d{d}", flush=True)
+
+    def grads(width):
+        q, k, v, do = (torch.nn.functional.pad(t, (0, width - d)).cuda() for t in x.values())
+        parts = [t.requires_grad_(True) for t in (q, k, v)]
+        out = flash_attn_npu_v2.flash_attn_func(*parts, softmax_scale=d ** -0.5, causal=True)
+        return [t.detach()[..., :d].float().cpu() for t in (out, *torch.autograd.grad(out, parts, do))]
+
+    for name, got, want in zip(("out", "dq", "dk", "dv"), grads(d), grads(full)):
+        same = (got == want) | (got.isnan() & want.isnan())
+        assert bool(same.all()), f"{name}: {int((~same).sum())} elements differ, {int(got.isnan().sum())} NaN, {int(want.isnan().sum())} wanted"
