@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -233,6 +234,82 @@ fa_status_t validate(const fa_fwd_params* p, int kind) {
     return FA_OK;
 }
 
+// Keys that an item of bm packed rows sees: the longest item's and the mean
+// one's. Lengths that only the device knows are taken from totals and
+// capacities: ragged queries are as long as their mean, in self attention (where
+// the long sequences have most of the work) as the geometric mean of that and
+// the longest, and a cache is half filled past the new rows.
+struct SeenKeys {
+    double longest, mean;
+};
+SeenKeys seen_keys(const fa_fwd_params* p, int kind, const Plan& pl, int bm) {
+    const double most = kind == FA_KIND_VARLEN && !p->block_table ? p->seqlen_k : pl.kv_capacity;
+    double sq = p->cu_seqlens_q ? std::max(1.0, (double)p->total_q / p->batch) : std::max(1, p->seqlen_q);
+    double sk = most;
+    if (kind == FA_KIND_KVCACHE || p->block_table) sk = most > sq ? (sq + most) / 2 : most;
+    else if (p->cu_seqlens_q && p->seqlen_k <= p->seqlen_q) sk = sq = std::min(most, std::sqrt(sq * most));
+    SeenKeys r = {sk, p->is_causal ? std::max(sk - sq, 0.0) + std::min(sk, sq) / 2 : sk};
+    const double positions = (double)bm / pl.g;
+    double bound = most;
+    if (p->window_size_left >= 0 && (p->is_causal || p->window_size_right >= 0))
+        bound = (double)p->window_size_left + (p->is_causal ? 0 : p->window_size_right) + positions;
+    if (p->attention_chunk > 0) bound = std::min(bound, p->attention_chunk + positions);
+    r.longest = std::min(r.longest, bound);
+    r.mean = std::min(r.mean, bound);
+    return r;
+}
+
+// Prefill tiles of the pipelined kernel, 128 or 256 rows, or 0 for the general
+// kernel, which batches of short sequences keep: with one wave per SIMD nothing
+// covers the start of an item, so a short item costs more there. The figures are
+// those that lose least on ~1000 random calls (8 to 32 heads, 1 to 64 sequences
+// of 64 to 6000 keys, dense, cached and ragged): 1.5 % more time than the best of
+// the three, against 4 % with the pipelined kernel always, in tiles by how they
+// fill the CUs, where one call in five took 3 to 60 % more than on the general one.
+// us, general / 128 / 256 rows: D64 full B64 S291 H8 44 / 68 / 70; D128 full
+// B45 S94 H16/4 27 / 36 / 35, B3 S1024 H16 - / 49 / 41; causal B7 S1100 H16
+// - / 83 / 104, B4 S4096 H32/8 - / 638 / 534; ragged D128 full, 50 sequences of 71 on average,
+// H24/8 46 / 62 / 63.
+int prefill_tiles(const fa_fwd_params* p, int kind, const Plan& pl) {
+    const int cus = cu_count();
+    const bool f8 = p->dtype == FA_DTYPE_FP8_E4M3;
+    // the general kernel would split the keys of few items, at a merge's cost; a
+    // soft cap takes it longer (2 instructions more per score, and no room for them)
+    const bool general = !pl.allow_split && p->num_splits <= 1;
+    const double cap = p->softcap > 0.f ? 1.6 : 1.0;
+    if (p->cu_seqlens_q) {
+        struct Short {
+            double items, keys;  // items of the general kernel per CU from which, mean keys up to which it is the faster
+        };
+        const Short lim = f8 ? Short{1.75, 240} : pl.kd == 64 ? Short{1.25, 640} : pl.kd == 128 ? Short{0.75, 440} : Short{0.75, 128};
+        auto items = [&](int bm) { return ((double)p->total_q * pl.g / bm + 0.5 * p->batch) * pl.hk_eff / cus; };
+        if (general && items(pl.BM) >= lim.items && cap * seen_keys(p, kind, pl, pl.BM).mean <= lim.keys) return 0;
+        // a row of a 128-row tile costs about 9 / 8 of one of a 256-row tile, part tiles included
+        return pl.kd == 256 || std::max(items(128), 1.0) * 128 * 9 < std::max(items(256), 1.0) * 256 * 8 ? 128 : 256;
+    }
+    // Same lengths: passes over the CUs times start and keys of an item
+    struct Item {
+        double start, keys;  // of an item, and of 64 keys; unit: 64 keys of a 128-row item
+    };
+    struct Items {
+        Item general, r128, r256;
+    };
+    const Items it = f8             ? Items{{12.5, 4.1}, {10.5, 1}, {17.7, 1.62}}
+                     : pl.kd == 64  ? Items{{13.7, 3.73}, {12.2, 1}, {21.9, 1.6}}
+                     : pl.kd == 128 ? Items{{3.3, 4.5}, {14.2, 1}, {25.6, 1.64}}
+                                    : Items{{2.6, 3.8}, {17.2, 1}, {0, 0}};
+    auto items = [&](int bm) { return (double)p->batch * pl.hk_eff * ((pl.rows_max + bm - 1) / bm) / cus; };
+    auto cost = [&](int bm, Item i) {
+        const double n = items(bm);
+        const SeenKeys seen = seen_keys(p, kind, pl, bm);
+        // one pass lasts as long as its longest item; heavy and light items are paired over several
+        return std::max(1.0, 0.85 * std::ceil(n) + 0.15 * n) * (i.start + i.keys * (n <= 1 ? seen.longest : seen.mean) / 64);
+    };
+    const double c128 = cost(128, it.r128), c256 = pl.kd == 256 ? INFINITY : cost(256, it.r256);
+    if (general && items(pl.BM) >= 1 && cost(pl.BM, {it.general.start, cap * it.general.keys}) < std::min(c128, c256)) return 0;
+    return c128 < c256 ? 128 : 256;
+}
+
 void make_plan(const fa_fwd_params* p, int kind, Plan& pl) {
     pl.hk_eff = p->no_pack_gqa ? p->nheads : p->nheads_k;
     pl.g = p->nheads / pl.hk_eff;
@@ -307,23 +384,17 @@ void make_plan(const fa_fwd_params* p, int kind, Plan& pl) {
     if (pl.allow_split) off = align256(off + sizeof(float) * (size_t)pl.items_max * pl.BM * pl.kd);
     pl.pipe = !pl.decode && fa::prefill_pipe_takes(p->dtype, pl.kd, p->softmax_scale, p->softcap, p->alibi_slopes != nullptr,
                                               pl.rotary, p->k_row_stride, p->v_row_stride, p->block_table != nullptr, p->page_block_size);
+    const int tiles = pl.pipe ? prefill_tiles(p, kind, pl) : 0;
+    pl.pipe = tiles > 0;
     if (pl.pipe) {
-        // One workgroup per CU, whatever the call. Tiles of 128 rows instead of
-        // 256 where the smaller ones fill the CUs better (dense causal B3 S700
-        // H16/4 32 -> 23 us; B4 S4096 H32/8 with them 523 -> 632), and a split of the keys only
+        // One workgroup per CU, whatever the call, and a split of the keys only
         // where a sequence can be long: a split costs a merge launch (about 9
         // us) and its partial rows, a tile of 64 keys about 1 us. us, with the
         // 256-row tiles and 128-key chunks before: dense causal B2 S512 H16 D128
         // 34.5 -> 20.4, B1 S1024 H16 49 -> 27, B1 S2048 H8 58 -> 37; 64 new rows
         // onto 4096 keys, H32/8, 58 -> 31. The scratch above, sized for the
         // larger tiles and the shorter chunks, covers either.
-        auto tiles = [&](int bm) -> int64_t {  // items of a call with tiles of bm rows (ragged: about)
-            if (p->cu_seqlens_q) return ((int64_t)p->total_q * pl.g / bm + pb / 2 + 1) * pl.hk_eff;
-            return (int64_t)pb * pl.hk_eff * ((pl.rows_max + bm - 1) / bm);
-        };
-        // a row of a 128-row tile costs about 9 / 8 of one of a 256-row tile
-        auto cost = [&](int bm, int rate) { return std::max<int64_t>(tiles(bm), cus) * bm * rate; };
-        pl.BM = pl.kd == 256 || cost(128, 9) < cost(256, 8) ? 128 : 256;
+        pl.BM = tiles;
         pl.mt_max = std::max(1, (pl.rows_max + pl.BM - 1) / pl.BM);
         const int64_t base = (int64_t)pb * pl.hk_eff * pl.mt_max;
         const int keys = kind == FA_KIND_VARLEN && !p->block_table ? p->seqlen_k : pl.kv_capacity;

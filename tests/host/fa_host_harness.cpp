@@ -40,6 +40,7 @@ struct Launch {
     const float* lse;
     const int* seqlens;
     int grid_kv, grid_q;  // backward
+    int pipe, tile_rows;  // prefill
 };
 std::vector<Launch> g_launch;
 void rec(const char* k, int B, const void* q, const void* out, const float* lse, const int* sl) {
@@ -62,6 +63,8 @@ int bwd_key_block(int d) { return d > 128 ? 64 : d > 64 ? 128 : 256; }
 int bwd_row_block(int d) { return d > 128 ? 64 : 128; }
 hipError_t launch_fwd(const FwdArgs& a, int, int, int, hipStream_t) {
     rec("fwd", a.B, a.q, a.out, a.lse, a.seqlens_k);
+    g_launch.back().pipe = a.pipe;
+    g_launch.back().tile_rows = a.tile_rows;
     return hipSuccess;
 }
 hipError_t launch_merge(const FwdArgs& a, int, int, hipStream_t) {
@@ -244,6 +247,50 @@ int main() {
             cov += l.B;
         }
         EXPECT(cov == B, "bwd covered %d of %d", cov, B);
+    }
+
+    // which prefill kernel takes a call: batches of short sequences the general one (0), others the pipelined one in
+    // tiles of 128 or 256 rows; each the fastest of the three where it was measured
+    struct Route { int B, sq, h, hk, d, causal; float cap; int want; };
+    const Route routes[] = {
+        {64, 291, 8, 8, 64, 0, 0.f, 0},      {31, 661, 16, 4, 64, 0, 0.f, 0},   {45, 94, 16, 4, 128, 0, 0.f, 0},
+        {34, 140, 32, 32, 128, 0, 0.f, 0},   {20, 211, 32, 32, 128, 1, 0.f, 0}, {33, 115, 32, 32, 256, 0, 0.f, 0},
+        {16, 1567, 24, 8, 64, 0, 20.f, 256}, {2, 512, 16, 16, 128, 1, 0.f, 128}, {2, 1024, 16, 16, 128, 0, 0.f, 128},
+        {3, 1024, 16, 16, 128, 0, 0.f, 256}, {7, 1100, 16, 16, 128, 1, 0.f, 128}, {4, 4096, 32, 8, 128, 1, 0.f, 256},
+        {4, 4096, 32, 8, 64, 0, 0.f, 256},   {2, 4096, 16, 8, 256, 1, 0.f, 128},
+    };
+    for (const Route& x : routes) {
+        fa_fwd_params p = base(x.B, x.sq, x.h, x.hk, x.d, x.sq);
+        p.is_causal = x.causal;
+        p.softcap = x.cap;
+        size_t ws = 0;
+        EXPECT(fa_fwd_workspace_size(&p, FA_KIND_DENSE, &ws) == FA_OK, "route: %s", fa_last_error());
+        p.workspace = (void*)0x10000000;
+        p.workspace_bytes = ws;
+        g_launch.clear();
+        EXPECT(fa_mha_fwd(&p, nullptr) == FA_OK && !g_launch.empty(), "route: %s", fa_last_error());
+        if (g_launch.empty()) continue;
+        const int got = g_launch[0].pipe ? g_launch[0].tile_rows : 0;
+        EXPECT(got == x.want, "B%d S%d H%d/%d D%d causal %d cap %g: route %d, not %d", x.B, x.sq, x.h, x.hk, x.d, x.causal,
+               x.cap, got, x.want);
+    }
+
+    // ragged self attention: by the sequences' mean and longest length
+    struct Ragged1 { int B, total, longest, h, hk, d, causal, general; };
+    for (const Ragged1& x : {Ragged1{50, 3537, 174, 24, 8, 128, 0, 1}, Ragged1{55, 6258, 257, 32, 8, 64, 0, 1},
+                             Ragged1{24, 12688, 2042, 16, 8, 128, 1, 0}, Ragged1{8, 16000, 3000, 16, 4, 64, 1, 0},
+                             Ragged1{2, 300, 200, 8, 8, 128, 0, 0}}) {
+        fa_fwd_params p = base(x.B, x.longest, x.h, x.hk, x.d, x.longest);
+        p.is_causal = x.causal;
+        p.total_q = x.total;
+        p.cu_seqlens_q = p.cu_seqlens_k = (const int32_t*)0x600000;
+        size_t ws = 0;
+        EXPECT(fa_fwd_workspace_size(&p, FA_KIND_VARLEN, &ws) == FA_OK, "ragged route: %s", fa_last_error());
+        p.workspace = (void*)0x10000000;
+        p.workspace_bytes = ws;
+        g_launch.clear();
+        EXPECT(fa_mha_varlen_fwd(&p, nullptr) == FA_OK && !g_launch.empty(), "ragged route: %s", fa_last_error());
+        if (!g_launch.empty()) EXPECT(g_launch[0].pipe == !x.general, "ragged B%d longest %d: pipelined %d", x.B, x.longest, g_launch[0].pipe);
     }
 
     // a ragged backward's dK / dV workgroups follow the keys, also where there are few query rows: one per item
