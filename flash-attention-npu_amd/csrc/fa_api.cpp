@@ -728,6 +728,29 @@ fa_status_t validate_bwd(const fa_bwd_params* p, int kind) {
     return FA_OK;
 }
 
+// Where the backward kernels with one wave per SIMD are the faster, as in the
+// prefill (prefill_tiles): not on short sequences or narrow windows, whose items
+// have little more than their start. Over 1000 random calls (1 to 64 sequences of
+// 48 to 4000 positions, half with a window of 31 to 1024) the time with these lines
+// is 0.2 to 1.1 % above that of the better kernel each time; with the pipelined
+// kernels always, 1 to 4.3 %, and one call in seven over 3 % slower than before them.
+// Whole backward, us, general -> pipelined: dQ D64, 63 sequences of 134 on average,
+// H32/8 192 -> 255, B48 S310 H16/4 136 -> 153; D128, 50 x 46 positions x 87 keys, H24/8
+// 65 -> 74; above these lengths 5 to 30 % the other way. dK/dV, 34 sequences of 37, H16
+// 52 -> 61; from 100 rows on 8 % the other way at the median.
+void backward_kernels(const fa_bwd_params* p, int kd, int g, fa::BwdArgs& a) {
+    double positions = p->cu_seqlens_q ? (double)p->total_q / p->batch : p->seqlen_q;  // of a sequence, on average
+    double keys = p->cu_seqlens_q && p->seqlen_k <= p->seqlen_q ? std::min<double>(positions, p->seqlen_k) : p->seqlen_k;
+    const double items = p->nheads_k * (p->cu_seqlens_q ? (double)p->total_q * g / 128 + 0.5 * p->batch
+                                                        : (double)p->batch * (((int64_t)p->seqlen_q * g + 127) / 128));
+    if (a.wl >= 0 && a.wr >= 0) {
+        keys = std::min(keys, (double)a.wl + a.wr);
+        positions = std::min(positions, (double)a.wl + a.wr + 64);
+    }
+    a.pipe_dq = kd == 256 ? keys > 60 : keys > (kd == 64 ? 450 : 150) || items < cu_count();
+    a.pipe_kv = positions * g > 100;
+}
+
 // Like the forward, a batch above kMaxBatch runs as consecutive launches over
 // batch chunks (the backward's per-batch item prefix lives in LDS).
 fa_status_t run_backward(const fa_bwd_params* p, int kind, void* stream_v) {
@@ -807,6 +830,7 @@ fa_status_t run_backward(const fa_bwd_params* p, int kind, void* stream_v) {
         a.wl = wl;
         a.wr = wr;
         a.chunk = p->attention_chunk;
+        backward_kernels(p, kd, a.g, a);
         const int64_t gkv = (int64_t)nb * p->nheads_k * (((int64_t)p->seqlen_k + fa::bwd_key_block(kd) - 1) / fa::bwd_key_block(kd));
         const int bm = std::min(fa::bwd_row_block(kd), 128);  // the smaller of the two dQ kernels' row tiles
         const int64_t gq = (int64_t)nb * p->nheads_k * (((int64_t)p->seqlen_q * a.g + bm - 1) / bm);

@@ -849,9 +849,9 @@ __global__ void __launch_bounds__(BwCfg<HD>::QNT, 1) fa_bwd_dq_kernel(BwdArgs a)
 // chunk tests would slow down.
 template <int DT, int HD, bool BIAS>
 static void launch_bwd_t(const BwdArgs& a, int grid_kv, int grid_q, hipStream_t stream) {
-    if (bwd_dq_takes(a)) launch_bwd_dq(a, DT, HD, grid_q, stream);
+    if (a.pipe_dq && bwd_dq_takes(a)) launch_bwd_dq(a, DT, HD, grid_q, stream);
     else hipLaunchKernelGGL((fa_bwd_dq_kernel<DT, HD, BIAS>), dim3(grid_q), dim3(BwCfg<HD>::QNT), 0, stream, a);
-    if (HD == 128 && !BIAS && bwd_kv_takes(a))
+    if (HD == 128 && !BIAS && a.pipe_kv && bwd_kv_takes(a))
         launch_bwd_kv(a, DT, grid_kv, stream);
     else if (a.chunk > 0)
         hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DT, HD, true, true>), dim3(grid_kv), dim3(BwCfg<HD>::KNT), 0, stream, a);

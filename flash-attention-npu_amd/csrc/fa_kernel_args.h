@@ -138,6 +138,7 @@ struct BwdArgs {
     int total_q;        // varlen: rows of q
     int wl, wr;         // normalised window, -1 = unbounded, causal => wr = 0
     int chunk;          // attention_chunk, 0 = off
+    int pipe_dq, pipe_kv;  // the kernels of fa_bwd_dq.hip / fa_bwd_kv.hip are the faster at these sizes
 };
 
 struct KvPrepArgs {

@@ -41,6 +41,7 @@ struct Launch {
     const int* seqlens;
     int grid_kv, grid_q;  // backward
     int pipe, tile_rows;  // prefill
+    int pipe_dq, pipe_kv;  // backward
 };
 std::vector<Launch> g_launch;
 void rec(const char* k, int B, const void* q, const void* out, const float* lse, const int* sl) {
@@ -91,6 +92,8 @@ hipError_t launch_bwd(const BwdArgs& a, int, int, int grid_kv, int grid_q, hipSt
     rec("bwd", a.B, a.q, a.dq, a.lse, nullptr);
     g_launch.back().grid_kv = grid_kv;
     g_launch.back().grid_q = grid_q;
+    g_launch.back().pipe_dq = a.pipe_dq;
+    g_launch.back().pipe_kv = a.pipe_kv;
     return hipSuccess;
 }
 }  // namespace fa
@@ -295,13 +298,19 @@ int main() {
 
     // a ragged backward's dK / dV workgroups follow the keys, also where there are few query rows: one per item
     // of (sequence, kv head, key block), or at least as many as there are items or CUs
-    struct Ragged { int B, total_q, max_q, max_k, hk, d, want; };
+    // (0: any number), and short sequences keep the general kernels
+    struct Ragged { int B, total_q, max_q, max_k, hk, d, want, dq, kv; };
     const Ragged ragged[] = {
-        {4, 64, 16, 8192, 8, 128, 2048},   // 16 positions each onto 8192 keys
-        {1, 256, 256, 32768, 8, 128, 2048},
-        {2, 2, 1, 4096, 2, 256, 256},      // 64-key blocks
-        {2, 2064, 2048, 2048, 2, 128, 64}, // the short sequence of the rows may be the long one of the keys
-        {64, 2048, 32, 32, 1, 64, 64},
+        {4, 64, 16, 8192, 8, 128, 2048, 1, 0},   // 16 positions each onto 8192 keys
+        {1, 256, 256, 32768, 8, 128, 2048, 1, 1},
+        {2, 2, 1, 4096, 2, 256, 256, 1, 0},      // 64-key blocks
+        {2, 2064, 2048, 2048, 2, 128, 64, 1, 1}, // the short sequence of the rows may be the long one of the keys
+        {64, 2048, 32, 32, 1, 64, 64, 1, 0},     // items for a quarter of the CUs
+        {63, 8442, 300, 300, 32, 64, 0, 0, 1},
+        {50, 6500, 180, 180, 16, 128, 0, 0, 1},
+        {34, 1258, 60, 60, 16, 128, 0, 0, 0},
+        {30, 1080, 60, 60, 16, 256, 0, 0, 0},
+        {24, 12688, 2042, 2042, 16, 128, 0, 1, 1},
     };
     for (const Ragged& x : ragged) {
         fa_bwd_params b;
@@ -329,6 +338,9 @@ int main() {
         if (g_launch.size() == 1)
             EXPECT(g_launch[0].grid_kv >= x.want, "ragged bwd B=%d q=%d k=%d: %d dK/dV workgroups for %d items", x.B,
                    x.max_q, x.max_k, g_launch[0].grid_kv, x.want);
+        if (g_launch.size() == 1)
+            EXPECT(g_launch[0].pipe_dq == x.dq && g_launch[0].pipe_kv == x.kv, "ragged bwd B=%d q=%d k=%d D=%d: dQ %d, dK/dV %d", x.B,
+                   x.max_q, x.max_k, x.d, g_launch[0].pipe_dq, g_launch[0].pipe_kv);
     }
 
     // invalid and extreme inputs must be refused (or accepted) without UB
