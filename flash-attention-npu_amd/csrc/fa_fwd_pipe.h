@@ -221,6 +221,20 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             load_tile(2, 2, std::false_type{});
         }
 
+        // V rows of a tile outside [begin, end) are no keys of the item: made 0 once
+        // they are there, for 0 weight times an infinity of the repeated key is no
+        // number (e4m3 has none). As masked loads it cost the whole loop 2.5 %; so, 1 %
+        // where the last tile is a part one.
+        [[maybe_unused]] auto clear_v = [&](int buf, int begin, int end) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int r = C::RPL * (4 * wave + u) + lane / CH;
+                if (r < begin || r >= end) row_write(lds0 + TILE * buf + KT + wave * 4096 + 1024 * u + 16 * lane, u32x4{0u, 0u, 0u, 0u});
+            }
+        };
+        const int last_end = k_hi - base - (ntiles - 1) * BN;
+        const int part_tile = __builtin_amdgcn_readfirstlane(!F8 && last_end < BN ? ntiles - 1 : -1);
+
         [[maybe_unused]] float sc_v = 1.f;
         [[maybe_unused]] uint32_t flip = 0;
         if constexpr (F8) {
@@ -452,6 +466,9 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
         if (ntiles > 0) {
             using H0 = std::integral_constant<int, 0>;
             wait_loads<0>();  // (with the q rows, which the compiler waits for)
+            if constexpr (PAGED && !F8) {
+                if (k_lo > base) clear_v(0, k_lo - base, BN);
+            }
             __syncthreads();
             f32x16 s0[RB], s1[RB];
 #pragma unroll
@@ -552,7 +569,13 @@ __global__ void __launch_bounds__(NT, 1) fa_prefill_pipe_kernel(FwdArgs a) {
             // half and of the next tile's first
             for (int part = 0; part < 2; ++part) {
                 const int tm = part == 0 ? t1 : ntiles;
-                while (t < tm) tile(std::true_type{});
+                while (t < tm) {
+                    if (__builtin_expect(t == part_tile, 0)) {
+                        clear_v(nb == 0 ? NBUF - 1 : nb - 1, 0, last_end);
+                        __syncthreads();
+                    }
+                    tile(std::true_type{});
+                }
                 while (t + 1 < t2) tile(std::false_type{});
             }
         }

@@ -208,3 +208,26 @@ def test_window_past_the_cache(sq, page):
         print(f"case window {window} sq{sq} page{page}", flush=True)
         got, want = (flash_attn_npu_v2.flash_attn_with_kvcache(q, k, v, window_size=w, **more) for w in (window, same))
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("d", [64, 96, 128, 256])
+@pytest.mark.parametrize("page", [0, 64])
+def test_infinity_in_v(d, page):
+    """An infinity in V of the first or the last key that the rows see stays that infinity: the rows of a tile that
+    are no keys of the call are 0, not that key again (0 times infinity)."""
+    import flash_attn_npu_v2
+    q, k, v = inputs(d, torch.bfloat16, (1, 1, 36, d), (1, 256, 2, d), (1, 256, 2, d))
+    seen, left = 150, 129  # one position, keys 20 .. 149
+    v[0, seen - 1, :, 3] = float("inf")
+    v[0, seen - 1 - left, :, 5] = -float("inf")
+    kd, vd = k.cuda(), v.cuda()
+    more = {}
+    if page:
+        kd, vd = (x.reshape(-1, page, 2, d) for x in (kd, vd))
+        more["block_table"] = torch.arange(256 // page, dtype=torch.int32).view(1, -1).cuda()
+    print(f"case infinity in v d{d} page{page}", flush=True)
+    out = flash_attn_npu_v2.flash_attn_with_kvcache(
+        q.cuda(), kd, vd, cache_seqlens=torch.tensor([seen], dtype=torch.int32).cuda(), window_size=(left, 0),
+        causal=True, num_splits=1, **more).float().cpu()
+    assert bool((out[..., 3] == float("inf")).all()) and bool((out[..., 5] == -float("inf")).all())
+    assert bool(out[..., [i for i in range(d) if i not in (3, 5)]].isfinite().all())
