@@ -949,7 +949,7 @@ def main():
             r["attn_frac_mfma"] = r["attn_tflops"] / BF16_PEAK_TFLOPS
             r["roofline"] = {"bound": "mfma", "achieved": round(r["attn_tflops"], 1), "peak": BF16_PEAK_TFLOPS,
                              "unit": "TFLOP/s", "frac": round(r["attn_frac_mfma"], 4), "traffic": measured_traffic(name),
-                             "kernel": "fa_prefill_kernel", "kernel_us": round(t["attn_us"], 2),
+                             "kernel": "fa_prefill_pipe_kernel", "kernel_us": round(t["attn_us"], 2),
                              "algorithmic_flops": c["flops"]}
         if not args.no_cpu and name in ("c2", "c3", "c4", "c5"):
             r["cpu_baseline"], ref = cpu_baseline(c, torch)
