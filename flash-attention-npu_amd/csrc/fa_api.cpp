@@ -273,8 +273,8 @@ SeenKeys seen_keys(const fa_fwd_params* p, int kind, const Plan& pl, int bm) {
 int prefill_tiles(const fa_fwd_params* p, int kind, const Plan& pl) {
     const int cus = cu_count();
     const bool f8 = p->dtype == FA_DTYPE_FP8_E4M3;
-    // the general kernel would split the keys of few items, at a merge's cost; a
-    // soft cap takes it longer (2 instructions more per score, and no room for them)
+    // the general kernel would split the keys of few items, at a merge's cost; with a
+    // soft cap it is the slower from shorter keys on (capped calls were among the random ones)
     const bool general = !pl.allow_split && p->num_splits <= 1;
     const double cap = p->softcap > 0.f ? 1.6 : 1.0;
     if (p->cu_seqlens_q) {

@@ -1,6 +1,8 @@
 // fa_bwd.hip -- FlashAttention backward (dense / varlen) for gfx950 (MI355X).
 // dQ of most calls runs on fa_bwd_dq.hip (bwd_dq_takes), dK / dV of plain calls at
-// head dims 65..128 on fa_bwd_kv.hip (bwd_kv_takes); the kernels here keep the rest.
+// head dims 65..128 on fa_bwd_kv.hip (bwd_kv_takes); the kernels here keep the rest
+// and, where they are the faster, short sequences and narrow windows
+// (BwdArgs::pipe_dq, pipe_kv, set by backward_kernels in fa_api.cpp).
 //
 // Reference behaviour being reproduced (paths relative to the reference repo):
 //   mha_bwd / mha_varlen_bwd       csrc/arch22/flash_attn_npu_v2/flash_api.cpp:1063-1299

@@ -433,7 +433,7 @@ void launch_d(const BwdArgs& a, int d, int grid, hipStream_t stream) {
 
 }  // namespace
 
-// Which calls run here; the others keep the kernel of fa_bwd.hip. The rows of a
+// Which calls can run here; the others keep the kernel of fa_bwd.hip. The rows of a
 // tile (16 KB) have 32-bit byte offsets.
 bool bwd_dq_takes(const BwdArgs& a) {
     auto fits = [](int64_t si) { return si >= 0 && si < (1 << 22); };

@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(NT, 1) fa_bwd_kv_kernel(BwdArgs a) {
 
 }  // namespace
 
-// Which calls run here; the others keep the kernel of fa_bwd.hip.
+// Which calls can run here; the others keep the kernel of fa_bwd.hip.
 // The rows of a tile are BQ / g positions of all g heads, so g divides BQ; their
 // byte offsets within a tile are 32-bit; -lse / scale stays in range.
 bool bwd_kv_takes(const BwdArgs& a) {

@@ -3,7 +3,8 @@
 // log-sum-exp combine. Most calls run on the pipelined kernel (fa_fwd_pipe.h,
 // chosen by prefill_pipe_takes); the one here keeps those with ALiBi, a soft cap
 // together with rotary, a non-positive scale, pages that a 16 KB tile does not
-// divide, row strides of 2^22 elements and more, and FP8 outside head dims 65..128.
+// divide, row strides of 2^22 elements and more, FP8 outside head dims 65..128,
+// and batches of short sequences (prefill_tiles in fa_api.cpp).
 //
 // Reference behaviour being reproduced (paths relative to the reference repo):
 //   SplitFuse::FAInfer / runMainLoop  csrc/arch22/flash_attn_npu_v2/mha_fwd_kvcache.cpp:436-966

@@ -21,7 +21,8 @@
 // Without the softmax 785 us, with products alone 730 (of 920, another box).
 // Head dim 256 (32 rows per wave, 32-key tiles), window 1024 and soft cap, B2 S4096
 // H16/8: 281 -> 190 us; head dim 64 (bound by the softmax, whose share of the
-// products is twice as large), B8 S1025 H16 fp16: 102 -> 97.
+// products is twice as large), B8 S1025 H16 fp16: 102 -> 97 (then 4 more for the
+// part tile that every item ends in, clear_v).
 #pragma once
 #include "fa_fwd.h"
 #include "fa_pipe.h"

@@ -88,11 +88,11 @@ struct FwdArgs {
     // head has its own (Hk = H, g = 1)
     int kvdiv;
     int tile_rows;      // prefill: packed rows per work tile
-    int pipe;           // prefill: runs on the pipelined kernel (prefill_pipe_takes)
+    int pipe;           // prefill: runs on the pipelined kernel
 };
 
-// Which prefill calls run on the pipelined kernel (fa_fwd_pipe.h); the others
-// keep the kernel of fa_fwd.hip. d: kernel head dim; dtype 0 / 1 / 3: fp16 / bf16 /
+// Which prefill calls can run on the pipelined kernel (fa_fwd_pipe.h); the others,
+// and those that are faster there, keep the kernel of fa_fwd.hip. d: kernel head dim; dtype 0 / 1 / 3: fp16 / bf16 /
 // e4m3 (at head dim 128).
 // The rows of a tile (16 KB) have 32-bit byte offsets, and a paged tile lies in
 // one page.

@@ -81,7 +81,7 @@ def hazards(lines):
     (["s_nop 3", "s_mov_b32 m0, s9"], True),
     (["s_nop 4"], False),
 ])
-def test_checker(between, early):
+def test_scan_finds_early_loads(between, early):
     lines = ["v_readfirstlane_b32 s7, v1", *between, "global_load_lds_dwordx4 v2, s[6:7] offset:1024 // 0:"]
     loads, bad = hazards(lines)
     assert loads == 1 and len(bad) == early
