@@ -398,7 +398,12 @@ void make_plan(const fa_fwd_params* p, int kind, Plan& pl) {
         pl.mt_max = std::max(1, (pl.rows_max + pl.BM - 1) / pl.BM);
         const int64_t base = (int64_t)pb * pl.hk_eff * pl.mt_max;
         const int keys = kind == FA_KIND_VARLEN && !p->block_table ? p->seqlen_k : pl.kv_capacity;
-        if (p->num_splits == 0 && keys <= kSplitKeys) pl.allow_split = false;
+        // Equal items on more than half of the CUs: two pieces of each would take two
+        // passes. us, split -> not (general kernel, split): full mask B1 S2550 H12 D128
+        // 99 -> 60 (82), S2646 H16/4 105 -> 81 (94), D64 B7 263 x 3377 H12 85 -> 47 (72);
+        // B1 S2048 H8, half of the CUs, is 39 split.
+        const bool equal = kind == FA_KIND_DENSE && !p->is_causal && p->window_size_left < 0 && p->window_size_right < 0 && p->attention_chunk == 0;
+        if (p->num_splits == 0 && (keys <= kSplitKeys || (equal && 2 * base > cus))) pl.allow_split = false;
         pl.min_chunk = kSplitKeys / 2;
         pl.target_items = cus;
         if (pl.allow_split || !p->cu_seqlens_q) pl.grid = cus;

@@ -278,6 +278,21 @@ int main() {
                x.cap, got, x.want);
     }
 
+    // equal items on more than half of the CUs are not split (no merge launch), fewer or unequal ones are
+    struct Split { int B, s, h, d, causal, launches; };
+    for (const Split& x : {Split{1, 2550, 12, 128, 0, 1}, Split{1, 2048, 12, 64, 0, 1}, Split{2, 1200, 8, 256, 0, 1},
+                           Split{1, 2048, 8, 128, 0, 2}, Split{1, 2550, 12, 128, 1, 2}}) {
+        fa_fwd_params p = base(x.B, x.s, x.h, x.h, x.d, x.s);
+        p.is_causal = x.causal;
+        size_t ws = 0;
+        EXPECT(fa_fwd_workspace_size(&p, FA_KIND_DENSE, &ws) == FA_OK, "split: %s", fa_last_error());
+        p.workspace = (void*)0x10000000;
+        p.workspace_bytes = ws;
+        g_launch.clear();
+        EXPECT(fa_mha_fwd(&p, nullptr) == FA_OK && (int)g_launch.size() == x.launches, "split B%d S%d H%d D%d causal %d: %zu launches, not %d",
+               x.B, x.s, x.h, x.d, x.causal, g_launch.size(), x.launches);
+    }
+
     // ragged self attention: by the sequences' mean and longest length
     struct Ragged1 { int B, total, longest, h, hk, d, causal, general; };
     for (const Ragged1& x : {Ragged1{50, 3537, 174, 24, 8, 128, 0, 1}, Ragged1{55, 6258, 257, 32, 8, 64, 0, 1},
